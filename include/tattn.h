@@ -115,6 +115,18 @@ int tattn_bwd(const void* q, const void* k, const void* v, const void* o, const 
               int dtype, int causal, float sm_scale, int config_id, void* stream);
 
 /*
+ * tattn_bwd with the gradients in a layout of their own: q, k, v, o and do share `strides`, dq, dk
+ * and dv share `grad_strides`. The backward then reads activations where they lie (a token-major
+ * view, say) and writes contiguous gradients, where the reference first copies its inputs
+ * contiguous (api.py:111). Same results bit for bit as tattn_bwd on contiguous copies.
+ */
+int tattn_bwd_layouts(const void* q, const void* k, const void* v, const void* o, const void* dout,
+                      void* dq, void* dk, void* dv, const float* m, float* delta,
+                      const int64_t strides[4], const int64_t grad_strides[4],
+                      int64_t Z, int64_t H, int64_t N, int64_t D, int dtype, int causal,
+                      float sm_scale, int config_id, void* stream);
+
+/*
  * tattn_bwd without the delta argument and without any allocation: delta lives in a static
  * device array of the library (16 MiB per GPU, held until the process ends), so the caller
  * passes only inputs and outputs. No counterpart in the reference: it is for callers that

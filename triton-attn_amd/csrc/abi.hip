@@ -278,7 +278,7 @@ static int bwd_common(BwdParams& p, const int64_t strides[4], int64_t Z, int64_t
   int rc;
   if ((rc = check_shape(Z, H, N, D, dtype))) return rc;
   if (!strides) return set_error(TATTN_E_ARG, "strides are null");
-  p.s[0] = strides[0]; p.s[1] = strides[1]; p.s[2] = strides[2];
+  for (int i = 0; i < 3; ++i) p.s[i] = p.so[i] = strides[i];
   p.Z = (int32_t)Z; p.H = (int32_t)H; p.N = (int32_t)N;
   p.c = sm_scale * kLog2e;
   p.scale = sm_scale;
@@ -353,16 +353,17 @@ int tattn_bwd_dq(const void* q, const void* k, const void* v, const void* dout, 
 // anything is enqueued, so a nonzero return from tattn_bwd means no work was launched.
 static int bwd_prepare(BwdParams& p, int* dk_id, int* dq_id, bool* fuse, const void* q, const void* k,
                        const void* v, const void* o, const void* dout, void* dq, void* dk, void* dv, const float* m,
-                       float* delta, const int64_t strides[4], int64_t Z, int64_t H, int64_t N, int64_t D,
-                       int dtype, int causal, float sm_scale, int config_id) {
+                       float* delta, const int64_t strides[4], const int64_t grad_strides[4], int64_t Z,
+                       int64_t H, int64_t N, int64_t D, int dtype, int causal, float sm_scale, int config_id) {
   int rc;
   if ((rc = bwd_common(p, strides, Z, H, N, D, dtype, sm_scale))) return rc;
   const int sz = dtype == TATTN_F32 ? 4 : 2;
   if ((rc = check_tensor("q", q, strides, sz)) || (rc = check_tensor("k", k, strides, sz)) ||
       (rc = check_tensor("v", v, strides, sz)) || (rc = check_tensor("o", o, strides, sz)) ||
-      (rc = check_tensor("do", dout, strides, sz)) || (rc = check_tensor("dq", dq, strides, sz)) ||
-      (rc = check_tensor("dk", dk, strides, sz)) || (rc = check_tensor("dv", dv, strides, sz)))
+      (rc = check_tensor("do", dout, strides, sz)) || (rc = check_tensor("dq", dq, grad_strides, sz)) ||
+      (rc = check_tensor("dk", dk, grad_strides, sz)) || (rc = check_tensor("dv", dv, grad_strides, sz)))
     return rc;
+  for (int i = 0; i < 3; ++i) p.so[i] = grad_strides[i];
   if (!m || !delta) return set_error(TATTN_E_ARG, "m and delta must not be null");
   if (config_id >= 0) {
     // One id for both kernels, as the reference's `config=` (api.py:124-145): it must exist in both tables.
@@ -382,14 +383,15 @@ static int bwd_prepare(BwdParams& p, int* dk_id, int* dq_id, bool* fuse, const v
   return TATTN_OK;
 }
 
-int tattn_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout, void* dq, void* dk,
-              void* dv, const float* m, float* delta, const int64_t strides[4], int64_t Z, int64_t H, int64_t N,
-              int64_t D, int dtype, int causal, float sm_scale, int config_id, void* stream) {
+int tattn_bwd_layouts(const void* q, const void* k, const void* v, const void* o, const void* dout, void* dq,
+                      void* dk, void* dv, const float* m, float* delta, const int64_t strides[4],
+                      const int64_t grad_strides[4], int64_t Z, int64_t H, int64_t N, int64_t D, int dtype,
+                      int causal, float sm_scale, int config_id, void* stream) {
   BwdParams p{};
   int rc, dk_id = -1, dq_id = -1;
   bool fuse = false;
-  if ((rc = bwd_prepare(p, &dk_id, &dq_id, &fuse, q, k, v, o, dout, dq, dk, dv, m, delta, strides, Z, H, N, D,
-                        dtype, causal, sm_scale, config_id)))
+  if ((rc = bwd_prepare(p, &dk_id, &dq_id, &fuse, q, k, v, o, dout, dq, dk, dv, m, delta, strides, grad_strides,
+                        Z, H, N, D, dtype, causal, sm_scale, config_id)))
     return rc;
   const hipStream_t st = (hipStream_t)stream;
   if (fuse) {
@@ -401,6 +403,13 @@ int tattn_bwd(const void* q, const void* k, const void* v, const void* o, const 
   if ((rc = launch_bwd_preprocess(p, (int)D, dtype, st))) return rc;
   if ((rc = launch_bwd_dkdv(p, (int)D, dtype, causal != 0, dk_id, st))) return rc;
   return launch_bwd_dq(p, (int)D, dtype, causal != 0, dq_id, st);
+}
+
+int tattn_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout, void* dq, void* dk,
+              void* dv, const float* m, float* delta, const int64_t strides[4], int64_t Z, int64_t H, int64_t N,
+              int64_t D, int dtype, int causal, float sm_scale, int config_id, void* stream) {
+  return tattn_bwd_layouts(q, k, v, o, dout, dq, dk, dv, m, delta, strides, strides, Z, H, N, D, dtype, causal,
+                           sm_scale, config_id, stream);
 }
 
 int tattn_bwd_noalloc(const void* q, const void* k, const void* v, const void* o, const void* dout, void* dq,

@@ -343,8 +343,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void dkdv_kernel(const BwdParams p) {
   }
 
   // Store: C register r of lane holds key 8*(r/4) + 4*h2 + r%4 of tile t, column 32u + l32.
-  T* DKg = (T*)p.dk + hd.off;
-  T* DVg = (T*)p.dv + hd.off;
+  T* DKg = (T*)p.dk + slice_off(p.so, zh, p.H);
+  T* DVg = (T*)p.dv + slice_off(p.so, zh, p.H);
 #pragma unroll
   for (int t = 0; t < KTW; ++t)
 #pragma unroll
@@ -355,8 +355,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void dkdv_kernel(const BwdParams p) {
         for (int r = 0; r < 16; ++r) {
           const int key = kw0 + 32 * t + 8 * (r >> 2) + 4 * h2 + (r & 3);
           if (key < N) {
-            DKg[(int64_t)key * rs + d] = (T)(dk[t][u][r] * p.scale);
-            DVg[(int64_t)key * rs + d] = (T)dv[t][u][r];
+            DKg[(int64_t)key * p.so[2] + d] = (T)(dk[t][u][r] * p.scale);
+            DVg[(int64_t)key * p.so[2] + d] = (T)dv[t][u][r];
           }
         }
       }
@@ -538,12 +538,12 @@ __global__ __launch_bounds__(NW * 64, OCC) void dq_kernel(const BwdParams p) {
   }
 
   // dQ^T C layout: lane = query, register r = column 32u + 8*(r/4) + 4*h2 + r%4.
-  T* DQg = (T*)p.dq + hd.off;
+  T* DQg = (T*)p.dq + slice_off(p.so, zh, p.H);
 #pragma unroll
   for (int j = 0; j < QTW; ++j) {
     const int q = qw0 + 32 * j + l32;
     if (q < N) {
-      T* row = DQg + (int64_t)q * rs;
+      T* row = DQg + (int64_t)q * p.so[2];
 #pragma unroll
       for (int u = 0; u < C::DT; ++u)
 #pragma unroll

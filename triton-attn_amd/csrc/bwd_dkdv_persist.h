@@ -267,7 +267,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void dkdv_persist_kernel(const BwdPar
       const int row = j / CPRO, cc = j % CPRO;
       if (row < 32) {
         const u32x4 v = *reinterpret_cast<const TATTN_LDS u32x4*>((const TATTN_LDS char*)wb + row * RB + 16 * cc);
-        st16_stream(dst + (int64_t)(kw0 + row) * rs + 8 * cc, v);
+        st16_stream(dst + (int64_t)(kw0 + row) * p.so[2] + 8 * cc, v);
       }
     }
   };
@@ -385,7 +385,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void dkdv_persist_kernel(const BwdPar
       }
     }
     {
-      const int64_t hoff = (int64_t)(zh_cur / p.H) * p.s[0] + (int64_t)(zh_cur % p.H) * p.s[1];
+      const int64_t hoff = slice_off(p.so, zh_cur, p.H);
       store_tile(dk, p.scale, (T*)p.dk + hoff, kv_w);
       store_tile(dv, 1.0f, (T*)p.dv + hoff, kv_w + TILE);
     }

@@ -289,8 +289,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void dq_persist_kernel(const BwdParam
             *reinterpret_cast<TATTN_LDS V4*>(wt + Swz<D>::addr(rl, 2 * d0)) = x;
           }
         }
-      const int64_t hoff = (int64_t)(zh / p.H) * p.s[0] + (int64_t)(zh % p.H) * p.s[1];
-      T* base = (T*)p.dq + hoff + (int64_t)(qb * BMQ + 32 * w) * rs;
+      T* base = (T*)p.dq + slice_off(p.so, zh, p.H) + (int64_t)(qb * BMQ + 32 * w) * p.so[2];
       constexpr int CPRO = D / 8;  // 16-byte chunks of a row
       int ln = lane;
       asm volatile("" : "+v"(ln));
@@ -299,7 +298,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void dq_persist_kernel(const BwdParam
         const int j = ln + 64 * it;
         const int row = j / CPRO, cc = j % CPRO;
         const u32x4 v = *reinterpret_cast<const TATTN_LDS u32x4*>(wt + Swz<D>::addr(row, 16 * cc));
-        st16_stream(base + (int64_t)row * rs + 8 * cc, v);
+        st16_stream(base + (int64_t)row * p.so[2] + 8 * cc, v);
       }
     }
     if (!more) break;

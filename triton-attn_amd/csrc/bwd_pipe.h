@@ -340,8 +340,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void dkdv_pipe_kernel(const BwdParams
   constexpr int SPW = (32 * CPRO + 63) / 64;  // chunk stores per lane and tile
   static_assert(NW * 32 * RB <= B::NST * STAGE, "store blocks fit the ring");
   char* wb = smem + w * 32 * RB;
-  T* DK = (T*)p.dk + hoff;
-  T* DV = (T*)p.dv + hoff;
+  T* DK = (T*)p.dk + slice_off(p.so, zh, p.H);
+  T* DV = (T*)p.dv + slice_off(p.so, zh, p.H);
   // The lane index is recomputed here (mbcnt) rather than kept live across the main loop, which
   // runs at the register limit.
   const int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
@@ -361,7 +361,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void dkdv_pipe_kernel(const BwdParams
       const int key = key0 + row;
       if (row < 32 && key < N) {
         const u32x4 v = *reinterpret_cast<const TATTN_LDS u32x4*>((const TATTN_LDS char*)wb + row * RB + 16 * cc);
-        st16_stream(dst + (int64_t)key * rs + 8 * cc, v);
+        st16_stream(dst + (int64_t)key * p.so[2] + 8 * cc, v);
       }
     }
   };
@@ -585,7 +585,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void dq_pipe_kernel(const BwdParams p
   if (wave_steps == nsteps && nsteps > 0) dq_mma(ea, (nsteps - 1) & 3);
 
   if (q < N) {
-    T* row = (T*)p.dq + hoff + (int64_t)q * rs;
+    T* row = (T*)p.dq + slice_off(p.so, zh, p.H) + (int64_t)q * p.so[2];
 #pragma unroll
     for (int u = 0; u < DT; ++u)
 #pragma unroll

@@ -304,7 +304,7 @@ __global__ __launch_bounds__(512, 2) void dkdv_split_kernel(const BwdParams p) {
   const int l32e = ln & 31, h2e = ln >> 5;
   char* wb = smem + wu * 32 * RB;
   const float mul = role_b ? p.scale : 1.0f;
-  T* dst = (T*)(role_b ? p.dk : p.dv) + hoff;
+  T* dst = (T*)(role_b ? p.dk : p.dv) + slice_off(p.so, zh, p.H);
   {
     TATTN_LDS T* wl = (TATTN_LDS T*)((TATTN_LDS char*)wb + 4 * h2e * RB) + l32e;
 #pragma unroll
@@ -320,7 +320,7 @@ __global__ __launch_bounds__(512, 2) void dkdv_split_kernel(const BwdParams p) {
       const int key = kw0 + row;
       if (row < 32 && key < N) {
         const u32x4 v = *reinterpret_cast<const TATTN_LDS u32x4*>((const TATTN_LDS char*)wb + row * RB + 16 * cc);
-        st16_stream(dst + (int64_t)key * rs + 8 * cc, v);
+        st16_stream(dst + (int64_t)key * p.so[2] + 8 * cc, v);
       }
     }
   }
@@ -600,7 +600,7 @@ __global__ __launch_bounds__(512, 2) void dq_split_kernel(const BwdParams p) {
       const int row = j / CPRO, cc = j % CPRO;
       const int qe = qw0 + row;
       const u32x4 v = *reinterpret_cast<const TATTN_LDS u32x4*>(wt + Swz<D>::addr(row, 16 * cc));
-      if (qe < N) st16_stream((T*)p.dq + hoff + (int64_t)qe * rs + 8 * cc, v);
+      if (qe < N) st16_stream((T*)p.dq + slice_off(p.so, zh, p.H) + (int64_t)qe * p.so[2] + 8 * cc, v);
     }
   }
 }

@@ -204,7 +204,8 @@ struct BwdParams {
   void* dv;
   const float* m;
   float* delta;
-  int64_t s[3];  // shared (z, h, n) strides in elements; d stride is 1
+  int64_t s[3];   // (z, h, n) strides in elements shared by q, k, v, o, dO; d stride is 1
+  int64_t so[3];  // (z, h, n) strides shared by dq, dk, dv
   int32_t Z, H, N;
   int32_t n_blocks;
   float c;      // sm_scale * log2(e)
@@ -212,6 +213,11 @@ struct BwdParams {
   int32_t items_x, gx, cus;  // persistent kernels: items per XCD, workgroups per XCD, CUs
   int32_t fuse_delta;        // dQ computes delta from O and dO itself and stores it (no preprocess)
 };
+
+// Element offset of slice zh = z * H + h in the backward's inputs (s) or its gradients (so).
+__device__ __forceinline__ int64_t slice_off(const int64_t (&st)[3], int zh, int H) {
+  return (int64_t)(zh / H) * st[0] + (int64_t)(zh % H) * st[1];
+}
 
 // Bytes spanned by rows [0, N) of a row-strided slice: every offset of a valid element is below
 // it and every offset of row N or later is at or above it.

@@ -101,6 +101,28 @@ def _kernel_layout(t: torch.Tensor) -> torch.Tensor:
     return t if ok else t.contiguous()
 
 
+def _one_layout(q: torch.Tensor, *others: torch.Tensor) -> bool:
+    """Whether the backward reads these tensors where they lie: one (z, h, n) layout for all of
+    them that the kernels take (`_kernel_layout`), with slices that 32-bit offsets span (beyond
+    that the kernels for wide slices are slower than a contiguous copy). Token-major activations,
+    the output that inherits their layout and its gradient are the usual case; the five copies
+    that the reference's backward starts with (api.py:111) took 78 us of 334 at 11 x 12 x 1500
+    tokens x 64 in fp16, forward + backward, and 106 us of 721 at 2 x 16 x 4096 x 128 in bf16."""
+    st = q.stride()
+    ptrs = q.data_ptr()
+    for t in others:
+        if t.stride() != st:
+            return False
+        ptrs |= t.data_ptr()
+    size = q.element_size()
+    return (
+        ptrs % 16 == 0
+        and st[3] == 1
+        and (st[0] * size) % 16 == 0 and (st[1] * size) % 16 == 0 and (st[2] * size) % 16 == 0
+        and (q.shape[2] + 127) * st[2] * size < 1 << 31
+    )
+
+
 def _resolve(kernel: int, d: int, dtype: torch.dtype, config: Config, causal: bool, n: int) -> int:
     """Maps the reference-style `config=` to a table index: None -> the library's pick; an int is
     the index; a dict may give "id" or any of block_m / block_n / waves / tiles / kind / ring
@@ -239,22 +261,25 @@ def _backward(
     z, h, n, d = q.shape
     if do.dtype != q.dtype:
         do = do.to(q.dtype)
-    q, k, v, do, o = q.contiguous(), k.contiguous(), v.contiguous(), do.contiguous(), o.contiguous()
+    whole = config is None and not _autotune  # one library call, which takes the inputs' own layout
+    if not (whole and _one_layout(q, k, v, do, o)):
+        q, k, v, do, o = q.contiguous(), k.contiguous(), v.contiguous(), do.contiguous(), o.contiguous()
     m = m.contiguous()
     delta = q.new_empty((z, h, n), dtype=torch.float32)
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    dq, dk, dv = q.new_empty(q.shape), q.new_empty(q.shape), q.new_empty(q.shape)
     if q.numel() == 0:
         return dq, dk, dv
     code = _DTYPES[q.dtype]
-    _, (st,) = _lib.stride_block(q)
-    if config is None and not _autotune:
+    if whole:
         # The whole backward in one library call: preprocess, dK/dV, dQ in stream order.
+        _, (st, gst) = _lib.stride_block(q, dq)
         with _on_device(q):
-            rc = lib.tattn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(),
-                               dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), m.data_ptr(), delta.data_ptr(), st,
-                               z, h, n, d, code, int(causal), float(scale), -1, _stream(q))
+            rc = lib.tattn_bwd_layouts(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(),
+                                       dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), m.data_ptr(), delta.data_ptr(),
+                                       st, gst, z, h, n, d, code, int(causal), float(scale), -1, _stream(q))
         _lib.check(rc, "tattn_bwd")
         return dq, dk, dv
+    _, (st,) = _lib.stride_block(q)
     if isinstance(config, dict) and ("dkdv" in config or "dq" in config):
         kid = _resolve(_lib.K_BWD_DKDV, d, q.dtype, config.get("dkdv"), causal, n)
         qid = _resolve(_lib.K_BWD_DQ, d, q.dtype, config.get("dq"), causal, n)
