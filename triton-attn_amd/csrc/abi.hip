@@ -270,6 +270,7 @@ int tattn_fwd(const void* q, const void* k, const void* v, void* o, float* m, co
   }
   p.Z = (int32_t)Z; p.H = (int32_t)H; p.N = (int32_t)N;
   p.c = sm_scale * kLog2e;
+  if (config_id < 0 && fwd_short_fits(p, dtype)) return launch_fwd_short(p, (int)D, dtype, causal != 0, (hipStream_t)stream);
   return launch_fwd(p, (int)D, dtype, causal != 0, id, (hipStream_t)stream);
 }
 
@@ -394,6 +395,7 @@ int tattn_bwd_layouts(const void* q, const void* k, const void* v, const void* o
                         Z, H, N, D, dtype, causal, sm_scale, config_id)))
     return rc;
   const hipStream_t st = (hipStream_t)stream;
+  if (config_id < 0 && bwd_short_fits(p, dtype)) return launch_bwd_short(p, (int)D, dtype, causal != 0, st);
   if (fuse) {
     BwdParams pq = p;
     pq.fuse_delta = 1;

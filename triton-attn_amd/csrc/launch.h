@@ -51,6 +51,19 @@ inline bool bwd_fits32(const BwdParams& p, int D) {
   return slice_bytes(p.N, p.s[2], D) + (uint64_t)p.s[2] * 128 < (1ull << 31);
 }
 
+// Short rows (short.hip): up to 128 rows of a slice in one workgroup's waves, the whole backward in
+// one launch. The rules check that a problem is one (16-bit, N within the limit) and that its row
+// offsets fit 32 bits.
+constexpr int kShortRows = 128;
+int launch_fwd_short(const FwdParams& p, int D, int dtype, bool causal, hipStream_t st);
+int launch_bwd_short(const BwdParams& p, int D, int dtype, bool causal, hipStream_t st);
+inline bool fwd_short_fits(const FwdParams& p, int dtype) {
+  return dtype != 1 && p.N <= kShortRows && (p.sk[2] | p.sv[2]) * 256 < (1ll << 30);
+}
+inline bool bwd_short_fits(const BwdParams& p, int dtype) {
+  return dtype != 1 && p.N <= kShortRows && p.s[2] * 256 < (1ll << 30);
+}
+
 // Compute units of the current device (cached per device).
 inline int device_cus() {
   static int cus[64] = {};
