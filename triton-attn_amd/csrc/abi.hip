@@ -2,6 +2,7 @@
 // device check, tile-table introspection and the entry points that enqueue the kernels.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -98,47 +99,142 @@ const TileEntry* config_entry(int kernel, int64_t D, int dtype, int id) {
   return nullptr;
 }
 
-// Table pick for a problem (index into the kernel's table), keyed like the reference's autotuner
-// on (sequence length, head dim, causal) (src/tattn/kernels.py:57-61), but static: the choices
-// below are the fastest entries measured on an MI355X at 16,384 tokens per batch, H=16. Entry 0
-// of each table is its general-purpose tile.
-// ZH = Z * H: the persistent forward entries are picked where they run the problem themselves.
-int pick_config(int kernel, int64_t D, int dtype, int causal, int64_t N, int64_t ZH) {
+// What a launch costs in rows of one CU: workgroups of `rows` rows are dealt to the 256 CUs, and the
+// CU with the most of them sets the time. `eff`: measured time per row against the fastest kernel
+// when the chip is full; `alone`: what a single workgroup of four waves on a CU (one wave per SIMD)
+// loses on top. Without a mask all workgroups of a launch are equal and this ranks the kernels
+// within a few percent (fp16, 1,000 to 8,192 row tiles, N = 500 to 12,345: e.g. forward, head dim 64,
+// 12 slices x 12,345 rows: 512-row blocks 1,024 CU rows 700 us, 256-row 768 569 us, 128-row 640
+// 530 us; 16 x 2,048: 512 59 us, 256 38 us, 128 26 us).
+double cu_rows(int64_t ZH, int64_t N, int rows, double eff, double alone = 1.0) {
+  const int64_t k = (ZH * ((N + rows - 1) / rows) + 255) / 256;
+  return (double)(k * rows) * eff * (k == 1 ? alone : 1.0);
+}
+
+// The same for coop.hip's kernels, whose prologue and final merge weigh on short rows (9 x 16 x 396:
+// 10-20% behind the block kernels where the row count alone puts them ahead).
+double coop_rows(int64_t ZH, int64_t N, double eff) { return cu_rows(ZH, N, 64, eff * (1.0 + 128.0 / (double)N)); }
+
+// The cheapest of a few candidates; the first wins ties.
+struct Cheapest {
+  double cost = 1e300;
+  int id = -1;
+  void offer(int i, double c) {
+    if (c < cost) cost = c, id = i;
+  }
+};
+
+// The kernels whose waves split the summed dimension (coop.hip), as a candidate.
+constexpr int kCoop = 1000;
+
+// Table pick for a problem (index into the kernel's table, or kCoop where `coop` allows it), keyed
+// like the reference's autotuner on (sequence length, head dim, causal) (src/tattn/kernels.py:57-61)
+// and on ZH = Z * H, but static: measured on an MI355X. Entry 0 of each table is its
+// general-purpose tile. Persistent entries are picked where they run the problem themselves.
+//
+// Causal launches are bound by their longest workgroups when the chip is not full: coop (a quarter
+// of the chain) up to a number of 32-row tiles, measured per kernel and head dim (us, coop against
+// the best other entry, N = 1,177 to 12,345):
+//   forward   64: 2,256 tiles 27.7 / 28.3, 6,000 134 / 126   128: 1,776 32.9 / 33.4, 2,256 46 / 42
+//             32: 6,000 82 / 83, 6,204 46 / 43
+//   dQ        64: 1,024 23 / 30, 1,760 95 / 118, 1,776 (N = 1,177) 31 / 26   128: 6,000 299 / 323, 6,204 170 / 167
+//             32: every size (8,192 tiles 51 / 53) from N = 768
+//   dK/dV     64: 1,024 31 / 45, 1,760 128 / 149, 1,776 (N = 1,177) 45 / 31   32: 4,632 299 / 314, 6,204 71 / 66, N = 384: 3,648 22 / 15
+//             128: never (its registers spill there)
+int pick_config(int kernel, int64_t D, int dtype, int causal, int64_t N, int64_t ZH, bool coop) {
   if (dtype == TATTN_F32) return 0;  // fp16 and bf16 share the picks
+  const int64_t tiles = ZH * ((N + 31) / 32);
+  Cheapest best;
   switch (kernel) {
-    case TATTN_K_FWD:  // persistent where it fits (D=64, 128); else 128-row blocks short, 256 / 512 long
+    case TATTN_K_FWD: {
+      // Fewer than 96 tiles keep the block kernels' single running max per row. The coop kernel's
+      // O and M of near one-hot rows (scores of +-100) are as close to float64 (M closer), but not
+      // the same bits, and on such rows one dS that rounds the other way moves a gradient by more
+      // than the flat flip allowance that the stress tests (2 x 1,024 rows) state. It would take
+      // 9 us where 1 x 1,024 x 64 takes 21.
+      coop = coop && tiles >= 96;
+      const int64_t coop_most = D == 64 ? 2304 : D == 128 ? 1800 : 6144;
+      if (causal && coop && tiles <= coop_most) return kCoop;
+      if (causal) {
+        if (D == 64) {
+          // Persistent, ring of 4: 4 x 2 from N = 2048 (from 4096 one pair of blocks per workgroup,
+          // time-sliced priority), 4 x 1 below (cold-cache medians, 16,384 tokens x 16 heads: N =
+          // 2048 4 x 2 3% faster since both store O as whole rows, N = 1024 4 x 1 2% faster).
+          const int pid = N < 2048 ? 5 : 7;
+          if (fwd_persist_fits(FwdTable<_Float16, 64>::e[pid], ZH, N, true)) return pid;
+        }
+        if (D == 128) {
+          const int pid = N >= 4096 ? 3 : 2;  // persistent 8 x 1 / 4 x 1; else 4 x 1 pipelined
+          return fwd_persist_fits(FwdTable<_Float16, 128>::e[pid], ZH, N, true) ? pid : 0;
+        }
+        // 128-row blocks; 256-row ones for long rows on a full chip.
+        return N >= 4096 && tiles >= 8192 ? 0 : 1;
+      }
       if (D == 64) {
-        // Persistent, ring of 4: 4 x 2 non-causal, and causal from N = 2048 (from 4096 one pair of
-        // blocks per workgroup, time-sliced priority); 4 x 1 causal below. Fastest at every
-        // benchmark length (cold-cache medians, 16,384 tokens x 16 heads; causal N = 2048: 4 x 2
-        // 3% faster than 4 x 1 since both store O as whole rows, N = 1024: 4 x 1 2% faster).
-        const int pid = causal && N < 2048 ? 5 : 7;
-        if (fwd_persist_fits(FwdTable<_Float16, 64>::e[pid], ZH, N, causal != 0)) return pid;
+        // Persistent 4 x 2 and 4 x 1 (ring of 4), pipelined 4 x 2, 8 x 2 from N = 4096, 4 x 1.
+        if (fwd_persist_fits(FwdTable<_Float16, 64>::e[7], ZH, N, false)) best.offer(7, cu_rows(ZH, N, 256, 0.95));
+        if (fwd_persist_fits(FwdTable<_Float16, 64>::e[5], ZH, N, false)) best.offer(5, cu_rows(ZH, N, 128, 1.07, 1.4));
+        best.offer(0, cu_rows(ZH, N, 256, 1.0));
+        if (N >= 4096) best.offer(3, cu_rows(ZH, N, 512, 0.99));
+        best.offer(1, cu_rows(ZH, N, 128, 1.06, 1.4));
+        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.4));
+      } else if (D == 128) {
+        // Persistent 8 x 1 from N = 2048, 4 x 1; pipelined 4 x 1.
+        if (N >= 2048 && fwd_persist_fits(FwdTable<_Float16, 128>::e[3], ZH, N, false))
+          best.offer(3, cu_rows(ZH, N, 256, 0.96));
+        if (fwd_persist_fits(FwdTable<_Float16, 128>::e[2], ZH, N, false)) best.offer(2, cu_rows(ZH, N, 128, 1.0, 1.1));
+        best.offer(0, cu_rows(ZH, N, 128, 1.02));
+        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.25));
+      } else {
+        best.offer(0, cu_rows(ZH, N, 256, 1.0));
+        best.offer(1, cu_rows(ZH, N, 128, D == 16 && N < 2048 ? 0.99 : 1.06, 1.4));
+        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.2));
       }
-      if (D == 128) {
-        // Persistent, ring of 4: 8 x 1 from N = 2048 (causal: 4096), 4 x 1 below; else 4 x 1
-        // pipelined.
-        const int pid = N >= (causal ? 4096 : 2048) ? 3 : 2;
-        if (fwd_persist_fits(FwdTable<_Float16, 128>::e[pid], ZH, N, causal != 0)) return pid;
-        return 0;
+      return best.id;
+    }
+    case TATTN_K_BWD_DKDV: {
+      const int64_t coop_most = D == 64 ? std::min<int64_t>(1800, N * 3 / 4) : D == 128 ? 0 : std::min<int64_t>(4800, N * 8 / 5);
+      if (causal && coop && tiles <= coop_most) return kCoop;
+      // Paired waves at head dim 128: two per SIMD, where one wave per tile needs all 512 registers.
+      if (D == 128) return 2;
+      if (causal) {
+        // Head dim 64: persistent 4 waves below N = 4096 where it fits, else pipelined, 8 waves (256
+        // keys) from N = 2048, 4 below; picked on the whole forward + backward (non-causal, the
+        // persistent entries lose there: the dQ pass leaves this kernel's inputs in the caches).
+        if (D != 64) return 0;
+        if (N < 4096 && bwd_persist_fits(DkdvTable<_Float16, 64>::e[5], ZH, N, true)) return 5;
+        return N >= 2048 ? 1 : 0;
       }
-      if (causal) return N >= 4096 ? 0 : 1;
-      if (D == 64) return N >= 4096 ? 3 : N >= 1024 ? 0 : 1;
-      return D == 16 && N < 2048 ? 1 : 0;
-    case TATTN_K_BWD_DKDV:  // causal N < 4096: persistent 4 waves where it fits; else pipelined, 8 waves
-                            // (256 keys), causal N < 2048: 4 waves (128 keys). Picked on the whole
-                            // forward + backward: there the persistent entries lose non-causal (the
-                            // dQ pass leaves this kernel's inputs in the caches).
-      if (D == 128) return 2;  // paired waves: two per SIMD, where one wave per tile needs all 512 registers
-      if (D != 64) return 0;
-      if (causal && N < 4096 && bwd_persist_fits(DkdvTable<_Float16, 64>::e[5], ZH, N, true)) return 5;
-      if (!causal) return 1;
-      return N >= 2048 ? 1 : 0;
-    case TATTN_K_BWD_DQ:  // persistent 4 waves where it fits; else 4 waves (8 for non-causal 2048 <= N < 8192)
-      if (D == 128) return 2;  // paired waves, as dK/dV
-      if (D != 64) return 0;
-      if (bwd_persist_fits(DqTable<_Float16, 64>::e[5], ZH, N, causal != 0)) return 5;
-      return !causal && N >= 2048 && N < 8192 ? 1 : 0;
+      if (D == 64) {
+        best.offer(1, cu_rows(ZH, N, 256, 1.0));
+        best.offer(0, cu_rows(ZH, N, 128, 1.35, 1.2));  // streams Q and dO past twice as many blocks
+        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.4 + 180.0 / (double)N));
+      } else {
+        best.offer(0, cu_rows(ZH, N, 128, 1.0, 1.4));
+        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.15));
+      }
+      return best.id;
+    }
+    case TATTN_K_BWD_DQ: {
+      // Head dims 16, 32: coop, except many short rows (16 x 16 x 384 causal: 13.6 against 12.7 us).
+      if (D < 64) return coop && (N >= (causal || D == 16 ? 768 : 448) || tiles <= N * 8 / 5) ? kCoop : 0;
+      const int64_t coop_most = D == 64 ? std::min<int64_t>(1800, N * 6 / 5) : 6000;
+      if (causal && coop && tiles <= coop_most) return kCoop;
+      if (D == 128) {  // paired waves, as dK/dV
+        if (causal) return 2;
+        best.offer(2, cu_rows(ZH, N, 128, 1.0));
+        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.05));
+        return best.id;
+      }
+      // Persistent 4 waves where it fits; pipelined 4 or 8 waves.
+      const bool persist = bwd_persist_fits(DqTable<_Float16, 64>::e[5], ZH, N, causal != 0);
+      if (causal) return persist ? 5 : 0;
+      if (persist) best.offer(5, cu_rows(ZH, N, 128, 0.95, 1.2));
+      best.offer(0, cu_rows(ZH, N, 128, 1.02, 1.2));
+      best.offer(1, cu_rows(ZH, N, 256, 1.06));
+      if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.25));
+      return best.id;
+    }
   }
   return 0;
 }
@@ -199,9 +295,23 @@ int check_shape(int64_t Z, int64_t H, int64_t N, int64_t D, int dtype) {
   return TATTN_OK;
 }
 
-int resolve(int kernel, int64_t D, int dtype, int causal, int64_t N, int64_t ZH, int id, int* out) {
+int run_fwd(const FwdParams& p, int D, int dtype, bool causal, int id, hipStream_t st) {
+  return id == kCoop ? launch_fwd_coop(p, D, dtype, causal, st) : launch_fwd(p, D, dtype, causal, id, st);
+}
+int run_dq(const BwdParams& p, int D, int dtype, bool causal, int id, hipStream_t st) {
+  return id == kCoop ? launch_dq_coop(p, D, dtype, causal, st) : launch_bwd_dq(p, D, dtype, causal, id, st);
+}
+int run_dkdv(const BwdParams& p, int D, int dtype, bool causal, int id, hipStream_t st) {
+  return id == kCoop ? launch_dkdv_coop(p, D, dtype, causal, st) : launch_bwd_dkdv(p, D, dtype, causal, id, st);
+}
+
+// A caller's table index, or the pick (coop: whether the problem meets coop.hip's preconditions).
+int resolve(int kernel, int64_t D, int dtype, int causal, int64_t N, int64_t ZH, int id, bool coop, int* out) {
   const int n = num_configs(kernel, D, dtype);
-  if (id < 0) id = pick_config(kernel, D, dtype, causal, N, ZH);
+  if (id < 0) {
+    *out = pick_config(kernel, D, dtype, causal, N, ZH, coop);
+    return TATTN_OK;
+  }
   if (id >= n) return set_error(TATTN_E_CONFIG, "config id %d out of range [0, %d)", id, n);
   *out = id;
   return TATTN_OK;
@@ -246,7 +356,7 @@ int tattn_config_desc(int kernel, int64_t D, int dtype, int config_id, tattn_con
 
 int tattn_pick_config(int kernel, int64_t D, int dtype, int causal, int64_t N) {
   if (num_configs(kernel, D, dtype) < 0) return set_error(TATTN_E_ARG, "no table for kernel %d, D=%lld", kernel, (long long)D), -1;
-  return pick_config(kernel, D, dtype, causal, N, 8);  // any Z * H that is a multiple of 8
+  return pick_config(kernel, D, dtype, causal, N, 1 << 16, false);  // a full chip, Z * H a multiple of 8
 }
 
 int tattn_fwd(const void* q, const void* k, const void* v, void* o, float* m, const int64_t q_strides[4],
@@ -260,9 +370,6 @@ int tattn_fwd(const void* q, const void* k, const void* v, void* o, float* m, co
       (rc = check_tensor("v", v, v_strides, sz)) || (rc = check_tensor("o", o, o_strides, sz)))
     return rc;
   // m may be null: the log-sum-exp is then not stored (no backward will follow).
-  int id;
-  if ((rc = resolve(TATTN_K_FWD, D, dtype, causal, N, Z * H, config_id, &id))) return rc;
-  if ((rc = device_check())) return rc;
   FwdParams p{};
   p.q = q; p.k = k; p.v = v; p.o = o; p.m = m;
   for (int i = 0; i < 3; ++i) {
@@ -270,8 +377,11 @@ int tattn_fwd(const void* q, const void* k, const void* v, void* o, float* m, co
   }
   p.Z = (int32_t)Z; p.H = (int32_t)H; p.N = (int32_t)N;
   p.c = sm_scale * kLog2e;
+  int id;
+  if ((rc = resolve(TATTN_K_FWD, D, dtype, causal, N, Z * H, config_id, fwd_coop_fits(p, (int)D, dtype), &id))) return rc;
+  if ((rc = device_check())) return rc;
   if (config_id < 0 && fwd_short_fits(p, dtype)) return launch_fwd_short(p, (int)D, dtype, causal != 0, (hipStream_t)stream);
-  return launch_fwd(p, (int)D, dtype, causal != 0, id, (hipStream_t)stream);
+  return run_fwd(p, (int)D, dtype, causal != 0, id, (hipStream_t)stream);
 }
 
 static int bwd_common(BwdParams& p, const int64_t strides[4], int64_t Z, int64_t H, int64_t N, int64_t D,
@@ -312,10 +422,10 @@ int tattn_bwd_dkdv(const void* q, const void* k, const void* v, const void* dout
     return rc;
   if (!m || !delta) return set_error(TATTN_E_ARG, "m and delta must not be null");
   int id;
-  if ((rc = resolve(TATTN_K_BWD_DKDV, D, dtype, causal, N, Z * H, config_id, &id))) return rc;
+  if ((rc = resolve(TATTN_K_BWD_DKDV, D, dtype, causal, N, Z * H, config_id, bwd_coop_fits(p, (int)D, dtype), &id))) return rc;
   if ((rc = device_check())) return rc;
   p.q = q; p.k = k; p.v = v; p.dout = dout; p.dk = dk; p.dv = dv; p.m = m; p.delta = const_cast<float*>(delta);
-  return launch_bwd_dkdv(p, (int)D, dtype, causal != 0, id, (hipStream_t)stream);
+  return run_dkdv(p, (int)D, dtype, causal != 0, id, (hipStream_t)stream);
 }
 
 // dQ; with o_fused (O, in the shared layout) the kernel computes delta = rowsum(dO * O) itself, in
@@ -333,14 +443,14 @@ static int bwd_dq_call(const void* q, const void* k, const void* v, const void* 
     return rc;
   if (!m || !delta) return set_error(TATTN_E_ARG, "m and delta must not be null");
   int id;
-  if ((rc = resolve(TATTN_K_BWD_DQ, D, dtype, causal, N, Z * H, config_id, &id))) return rc;
+  if ((rc = resolve(TATTN_K_BWD_DQ, D, dtype, causal, N, Z * H, config_id, bwd_coop_fits(p, (int)D, dtype), &id))) return rc;
   if ((rc = device_check())) return rc;
   p.q = q; p.k = k; p.v = v; p.dout = dout; p.dq = dq; p.m = m; p.delta = const_cast<float*>(delta);
   if (o_fused) {
     p.o = o_fused;
     p.fuse_delta = 1;
   }
-  return launch_bwd_dq(p, (int)D, dtype, causal != 0, id, (hipStream_t)stream);
+  return run_dq(p, (int)D, dtype, causal != 0, id, (hipStream_t)stream);
 }
 
 int tattn_bwd_dq(const void* q, const void* k, const void* v, const void* dout, void* dq, const float* m,
@@ -371,15 +481,16 @@ static int bwd_prepare(BwdParams& p, int* dk_id, int* dq_id, bool* fuse, const v
     if (config_id >= num_configs(TATTN_K_BWD_DKDV, D, dtype) || config_id >= num_configs(TATTN_K_BWD_DQ, D, dtype))
       return set_error(TATTN_E_CONFIG, "config id %d out of range for the backward tables", config_id);
   }
-  if ((rc = resolve(TATTN_K_BWD_DKDV, D, dtype, causal, N, Z * H, config_id, dk_id)) ||
-      (rc = resolve(TATTN_K_BWD_DQ, D, dtype, causal, N, Z * H, config_id, dq_id)))
+  const bool coop = bwd_coop_fits(p, (int)D, dtype);
+  if ((rc = resolve(TATTN_K_BWD_DKDV, D, dtype, causal, N, Z * H, config_id, coop, dk_id)) ||
+      (rc = resolve(TATTN_K_BWD_DQ, D, dtype, causal, N, Z * H, config_id, coop, dq_id)))
     return rc;
   if ((rc = device_check())) return rc;
   // When dQ runs a pipelined, persistent or paired-wave 16-bit kernel it computes delta itself
   // (same bits as the preprocess) and stores it: dQ, then dK/dV, two launches and no separate
   // pass over dO. Otherwise preprocess, dK/dV, dQ.
   const TileEntry* e = config_entry(TATTN_K_BWD_DQ, D, dtype, *dq_id);
-  *fuse = dtype != TATTN_F32 && e && e->pipe >= 1 && bwd_fits32(p, (int)D);
+  *fuse = *dq_id == kCoop || (dtype != TATTN_F32 && e && e->pipe >= 1 && bwd_fits32(p, (int)D));
   p.q = q; p.k = k; p.v = v; p.o = o; p.dout = dout; p.dq = dq; p.dk = dk; p.dv = dv; p.m = m; p.delta = delta;
   return TATTN_OK;
 }
@@ -399,12 +510,12 @@ int tattn_bwd_layouts(const void* q, const void* k, const void* v, const void* o
   if (fuse) {
     BwdParams pq = p;
     pq.fuse_delta = 1;
-    if ((rc = launch_bwd_dq(pq, (int)D, dtype, causal != 0, dq_id, st))) return rc;
-    return launch_bwd_dkdv(p, (int)D, dtype, causal != 0, dk_id, st);
+    if ((rc = run_dq(pq, (int)D, dtype, causal != 0, dq_id, st))) return rc;
+    return run_dkdv(p, (int)D, dtype, causal != 0, dk_id, st);
   }
   if ((rc = launch_bwd_preprocess(p, (int)D, dtype, st))) return rc;
-  if ((rc = launch_bwd_dkdv(p, (int)D, dtype, causal != 0, dk_id, st))) return rc;
-  return launch_bwd_dq(p, (int)D, dtype, causal != 0, dq_id, st);
+  if ((rc = run_dkdv(p, (int)D, dtype, causal != 0, dk_id, st))) return rc;
+  return run_dq(p, (int)D, dtype, causal != 0, dq_id, st);
 }
 
 int tattn_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout, void* dq, void* dk,

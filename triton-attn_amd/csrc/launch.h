@@ -64,6 +64,19 @@ inline bool bwd_short_fits(const BwdParams& p, int dtype) {
   return dtype != 1 && p.N <= kShortRows && p.s[2] * 256 < (1ll << 30);
 }
 
+// Waves of a workgroup split the summed dimension (coop.hip); 16-bit, slices that fit 32-bit
+// offsets, and for the forward a scale other than 0 (it hides keys at a score whose scaled value is -inf).
+int launch_fwd_coop(const FwdParams& p, int D, int dtype, bool causal, hipStream_t st);
+int launch_dq_coop(const BwdParams& p, int D, int dtype, bool causal, hipStream_t st);
+int launch_dkdv_coop(const BwdParams& p, int D, int dtype, bool causal, hipStream_t st);
+inline bool fwd_coop_fits(const FwdParams& p, int D, int dtype) {
+  return dtype != 1 && p.c != 0.0f && slice_bytes(p.N, p.sk[2], D) + (uint64_t)p.sk[2] * 128 < (1ull << 31) &&
+         slice_bytes(p.N, p.sv[2], D) + (uint64_t)p.sv[2] * 128 < (1ull << 31) && (p.sk[2] | p.sv[2]) < (1ll << 22);
+}
+inline bool bwd_coop_fits(const BwdParams& p, int D, int dtype) {
+  return dtype != 1 && bwd_fits32(p, D) && p.s[2] < (1ll << 22);
+}
+
 // Compute units of the current device (cached per device).
 inline int device_cus() {
   static int cus[64] = {};
