@@ -1,0 +1,111 @@
+"""The float32 kernels on split operands (the library's float32 picks) against float64 and against the
+block kernels on the float32 matrix instruction, at row counts around tiles, blocks and steps of every
+launch shape, in layouts, at scales and magnitudes, and with infinities."""
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BLOCKS = {"fwd": {"id": 0}, "bwd": {"dkdv": 0, "dq": 0}}
+
+
+def _rand(shape, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn(shape, device="cuda", generator=g)
+
+
+def _exact(q, k, v, do, causal, scale):
+    q, k, v, do = (t.double() for t in (q, k, v, do))
+    s = torch.matmul(q, k.transpose(-1, -2).contiguous()) * scale
+    if causal:
+        s = s.masked_fill(torch.ones(s.shape[-2:], dtype=torch.bool, device=s.device).triu(1), -math.inf)
+    p = torch.softmax(s, -1)
+    o = torch.matmul(p, v)
+    ds = (torch.matmul(do, v.transpose(-1, -2).contiguous()) - (do * o).sum(-1, keepdim=True)) * p * scale
+    return o, torch.matmul(ds, k), torch.matmul(ds.transpose(-1, -2).contiguous(), q), \
+        torch.matmul(p.transpose(-1, -2).contiguous(), do)
+
+
+def _run(q, k, v, do, causal, scale, blocks):
+    from tattn.api import _backward, _forward
+
+    o, m = _forward(q, k, v, causal, scale, config=BLOCKS["fwd"] if blocks else None)
+    return (o, *_backward(q, k, v, o, m, do, causal, scale, config=BLOCKS["bwd"] if blocks else None)), m
+
+
+def _compare(q, k, v, do, causal, scale):
+    """No further from float64 than the block kernels, up to a quarter and 2^-24 (both are a few
+    roundings of 2^-24 per sum; the order differs)."""
+    ref = _exact(q, k, v, do, causal, scale)
+    got, m = _run(q, k, v, do, causal, scale, False)
+    old, mb = _run(q, k, v, do, causal, scale, True)
+    for name, a, b, r in zip(("o", "dq", "dk", "dv"), got, old, ref):
+        size = r.norm().item()
+        ea, eb = (a.double() - r).norm().item(), (b.double() - r).norm().item()
+        assert ea <= 1.25 * eb + 2.0 ** -24 * size, (name, ea / size, eb / size)
+    # |scores| and their float32 sums: a few units in the last place of the largest, in log2.
+    assert (m - mb).abs().max().item() <= 1e-6 * (1 + mb.abs().max().item())
+    again, _ = _run(q, k, v, do, causal, scale, False)
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [16, 32, 64, 128])
+@pytest.mark.parametrize("z,h,n", [(2, 3, 2), (40, 16, 31), (40, 16, 33), (2, 3, 64), (40, 16, 65), (5, 7, 127),
+                                   (32, 8, 129), (1, 5, 257), (16, 16, 260), (1, 16, 513), (3, 8, 1000)])
+def test_split_kernels_against_float64(z, h, n, d, causal):
+    _compare(*(_rand((z, h, n, d), n + s) for s in range(4)), causal, d ** -0.5)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("scale", [-0.125, 0.0, 0.5])
+def test_scales(scale, causal):
+    _compare(*(_rand((2, 8, 300, 64), 50 + s) for s in range(4)), causal, scale)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_layouts(causal):
+    """Token-major, interleaved, and broadcast key / value views."""
+    _compare(*(_rand((2, 200, 8, 64), 70 + s).transpose(1, 2) for s in range(4)), causal, 0.125)
+    _compare(*(t.transpose(1, 2) for t in _rand((2, 200, 4, 8, 64), 80).unbind(2)), causal, 0.125)
+    q, do = (_rand((2, 8, 200, 64), 90 + s) for s in range(2))
+    k, v = (_rand((1, 1, 200, 64), 95 + s).expand(2, 8, 200, 64) for s in range(2))
+    _compare(q, k, v, do, causal, 0.125)
+
+
+@pytest.mark.parametrize("mag", [(1e-18, 1e18, 1.0, 1.0), (1.0, 1.0, 1e-37, 1.0), (1.0, 1.0, 1.0, 1e-36),
+                                 (1e-3, 1e3, 1e30, 1e-30), (1.0, 1.0, 1e36, 1e-20)])
+def test_magnitudes(mag):
+    """Values near both ends of the exponent range: no precision is lost to the planes' own range."""
+    _compare(*(_rand((2, 4, 150, 64), 100 + s) * x for s, x in enumerate(mag)), False, 0.125)
+
+
+@pytest.mark.parametrize("n", [40, 200, 600])
+@pytest.mark.parametrize("causal", [False, True])
+def test_infinities_and_nans_go_where_the_block_kernels_take_them(causal, n):
+    q, k, v, do = (_rand((2, 8, n, 64), 30 + s) for s in range(4))
+    q[0, 1, 17, 5] = float("nan")
+    k[0, 2, 3, 7] = float("-inf")  # hides key 3 from queries whose component is positive
+    v[0, 3, 9, 11] = float("inf")
+    v[1, 1, 6, 0] = float("nan")
+    do[1, 2, 8, 1] = float("inf")
+    v[1, 3, 1, 2] = 3e35
+    got, m = _run(q, k, v, do, causal, 0.125, False)
+    old, mb = _run(q, k, v, do, causal, 0.125, True)
+    for a, b in zip((*got, m), (*old, mb)):
+        assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.isinf(a), torch.isinf(b))
+        ok = torch.isfinite(b)
+        assert torch.equal(torch.sign(a[~ok & ~torch.isnan(b)]), torch.sign(b[~ok & ~torch.isnan(b)]))
+    assert torch.isfinite(got[0][0, 2][q[0, 2, :, 7] > 0]).all()
+
+
+def test_overlapping_rows_take_the_block_kernels():
+    """Keys that all share one row (row stride 0) are the block kernels' case: same bits."""
+    from tattn.api import _forward
+
+    q = _rand((2, 4, 100, 64), 1)
+    k, v = (_rand((2, 4, 1, 64), 2 + s).expand(2, 4, 100, 64) for s in range(2))
+    got, want = _forward(q, k, v, False, 0.125), _forward(q, k, v, False, 0.125, config={"id": 0})
+    assert all(torch.equal(a, b) for a, b in zip(got, want))

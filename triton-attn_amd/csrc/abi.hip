@@ -126,8 +126,11 @@ struct Cheapest {
 
 // The kernels whose waves split the summed dimension (coop.hip), as a candidate.
 constexpr int kCoop = 1000;
+// The float32 kernels on split operands (f32_split.hip).
+constexpr int kSplit = 1001;
 
-// Table pick for a problem (index into the kernel's table, or kCoop where `coop` allows it), keyed
+// Table pick for a problem (index into the kernel's table, or kCoop / kSplit where `own` says that
+// the problem meets the preconditions of coop.hip in 16 bits, of f32_split.hip in float32), keyed
 // like the reference's autotuner on (sequence length, head dim, causal) (src/tattn/kernels.py:57-61)
 // and on ZH = Z * H, but static: measured on an MI355X. Entry 0 of each table is its
 // general-purpose tile. Persistent entries are picked where they run the problem themselves.
@@ -141,8 +144,9 @@ constexpr int kCoop = 1000;
 //             32: every size (8,192 tiles 51 / 53) from N = 768
 //   dK/dV     64: 1,024 31 / 45, 1,760 128 / 149, 1,776 (N = 1,177) 45 / 31   32: 4,632 299 / 314, 6,204 71 / 66, N = 384: 3,648 22 / 15
 //             128: never (its registers spill there)
-int pick_config(int kernel, int64_t D, int dtype, int causal, int64_t N, int64_t ZH, bool coop) {
-  if (dtype == TATTN_F32) return 0;  // fp16 and bf16 share the picks
+int pick_config(int kernel, int64_t D, int dtype, int causal, int64_t N, int64_t ZH, bool own) {
+  if (dtype == TATTN_F32) return own ? kSplit : 0;  // fp16 and bf16 share the picks
+  bool coop = own;
   const int64_t tiles = ZH * ((N + 31) / 32);
   Cheapest best;
   switch (kernel) {
@@ -296,20 +300,26 @@ int check_shape(int64_t Z, int64_t H, int64_t N, int64_t D, int dtype) {
 }
 
 int run_fwd(const FwdParams& p, int D, int dtype, bool causal, int id, hipStream_t st) {
+  if (id == kSplit) return launch_fwd_f32(p, D, causal, st);
   return id == kCoop ? launch_fwd_coop(p, D, dtype, causal, st) : launch_fwd(p, D, dtype, causal, id, st);
 }
 int run_dq(const BwdParams& p, int D, int dtype, bool causal, int id, hipStream_t st) {
+  if (id == kSplit) return launch_dq_f32(p, D, causal, st);
   return id == kCoop ? launch_dq_coop(p, D, dtype, causal, st) : launch_bwd_dq(p, D, dtype, causal, id, st);
 }
 int run_dkdv(const BwdParams& p, int D, int dtype, bool causal, int id, hipStream_t st) {
+  if (id == kSplit) return launch_dkdv_f32(p, D, causal, st);
   return id == kCoop ? launch_dkdv_coop(p, D, dtype, causal, st) : launch_bwd_dkdv(p, D, dtype, causal, id, st);
 }
 
-// A caller's table index, or the pick (coop: whether the problem meets coop.hip's preconditions).
-int resolve(int kernel, int64_t D, int dtype, int causal, int64_t N, int64_t ZH, int id, bool coop, int* out) {
+bool fwd_own_fits(const FwdParams& p, int D, int dtype) { return dtype == TATTN_F32 ? fwd_f32_fits(p, D) : fwd_coop_fits(p, D, dtype); }
+bool bwd_own_fits(const BwdParams& p, int D, int dtype) { return dtype == TATTN_F32 ? bwd_f32_fits(p, D) : bwd_coop_fits(p, D, dtype); }
+
+// A caller's table index, or the pick (own: see pick_config).
+int resolve(int kernel, int64_t D, int dtype, int causal, int64_t N, int64_t ZH, int id, bool own, int* out) {
   const int n = num_configs(kernel, D, dtype);
   if (id < 0) {
-    *out = pick_config(kernel, D, dtype, causal, N, ZH, coop);
+    *out = pick_config(kernel, D, dtype, causal, N, ZH, own);
     return TATTN_OK;
   }
   if (id >= n) return set_error(TATTN_E_CONFIG, "config id %d out of range [0, %d)", id, n);
@@ -378,7 +388,7 @@ int tattn_fwd(const void* q, const void* k, const void* v, void* o, float* m, co
   p.Z = (int32_t)Z; p.H = (int32_t)H; p.N = (int32_t)N;
   p.c = sm_scale * kLog2e;
   int id;
-  if ((rc = resolve(TATTN_K_FWD, D, dtype, causal, N, Z * H, config_id, fwd_coop_fits(p, (int)D, dtype), &id))) return rc;
+  if ((rc = resolve(TATTN_K_FWD, D, dtype, causal, N, Z * H, config_id, fwd_own_fits(p, (int)D, dtype), &id))) return rc;
   if ((rc = device_check())) return rc;
   if (config_id < 0 && fwd_short_fits(p, dtype)) return launch_fwd_short(p, (int)D, dtype, causal != 0, (hipStream_t)stream);
   return run_fwd(p, (int)D, dtype, causal != 0, id, (hipStream_t)stream);
@@ -422,7 +432,7 @@ int tattn_bwd_dkdv(const void* q, const void* k, const void* v, const void* dout
     return rc;
   if (!m || !delta) return set_error(TATTN_E_ARG, "m and delta must not be null");
   int id;
-  if ((rc = resolve(TATTN_K_BWD_DKDV, D, dtype, causal, N, Z * H, config_id, bwd_coop_fits(p, (int)D, dtype), &id))) return rc;
+  if ((rc = resolve(TATTN_K_BWD_DKDV, D, dtype, causal, N, Z * H, config_id, bwd_own_fits(p, (int)D, dtype), &id))) return rc;
   if ((rc = device_check())) return rc;
   p.q = q; p.k = k; p.v = v; p.dout = dout; p.dk = dk; p.dv = dv; p.m = m; p.delta = const_cast<float*>(delta);
   return run_dkdv(p, (int)D, dtype, causal != 0, id, (hipStream_t)stream);
@@ -443,7 +453,7 @@ static int bwd_dq_call(const void* q, const void* k, const void* v, const void* 
     return rc;
   if (!m || !delta) return set_error(TATTN_E_ARG, "m and delta must not be null");
   int id;
-  if ((rc = resolve(TATTN_K_BWD_DQ, D, dtype, causal, N, Z * H, config_id, bwd_coop_fits(p, (int)D, dtype), &id))) return rc;
+  if ((rc = resolve(TATTN_K_BWD_DQ, D, dtype, causal, N, Z * H, config_id, bwd_own_fits(p, (int)D, dtype), &id))) return rc;
   if ((rc = device_check())) return rc;
   p.q = q; p.k = k; p.v = v; p.dout = dout; p.dq = dq; p.m = m; p.delta = const_cast<float*>(delta);
   if (o_fused) {
@@ -481,16 +491,16 @@ static int bwd_prepare(BwdParams& p, int* dk_id, int* dq_id, bool* fuse, const v
     if (config_id >= num_configs(TATTN_K_BWD_DKDV, D, dtype) || config_id >= num_configs(TATTN_K_BWD_DQ, D, dtype))
       return set_error(TATTN_E_CONFIG, "config id %d out of range for the backward tables", config_id);
   }
-  const bool coop = bwd_coop_fits(p, (int)D, dtype);
-  if ((rc = resolve(TATTN_K_BWD_DKDV, D, dtype, causal, N, Z * H, config_id, coop, dk_id)) ||
-      (rc = resolve(TATTN_K_BWD_DQ, D, dtype, causal, N, Z * H, config_id, coop, dq_id)))
+  const bool own = bwd_own_fits(p, (int)D, dtype);
+  if ((rc = resolve(TATTN_K_BWD_DKDV, D, dtype, causal, N, Z * H, config_id, own, dk_id)) ||
+      (rc = resolve(TATTN_K_BWD_DQ, D, dtype, causal, N, Z * H, config_id, own, dq_id)))
     return rc;
   if ((rc = device_check())) return rc;
-  // When dQ runs a pipelined, persistent or paired-wave 16-bit kernel it computes delta itself
+  // When dQ runs any kernel but the generic ones it computes delta itself
   // (same bits as the preprocess) and stores it: dQ, then dK/dV, two launches and no separate
   // pass over dO. Otherwise preprocess, dK/dV, dQ.
   const TileEntry* e = config_entry(TATTN_K_BWD_DQ, D, dtype, *dq_id);
-  *fuse = *dq_id == kCoop || (dtype != TATTN_F32 && e && e->pipe >= 1 && bwd_fits32(p, (int)D));
+  *fuse = *dq_id == kCoop || *dq_id == kSplit || (dtype != TATTN_F32 && e && e->pipe >= 1 && bwd_fits32(p, (int)D));
   p.q = q; p.k = k; p.v = v; p.o = o; p.dout = dout; p.dq = dq; p.dk = dk; p.dv = dv; p.m = m; p.delta = delta;
   return TATTN_OK;
 }
