@@ -21,10 +21,10 @@
 // are added through LDS at the end. Which RW and CS: pick_shape, below.
 //
 // What bounds it: matrix and vector work of the two waves of a SIMD barely overlap (forward of 4 x 16 x
-// 1,024 x 64: 98 thousand MFMA cycles and 88 thousand of vector issue per SIMD, of 187 thousand busy; 1.0
-// PFLOP/s of bf16 products). Vector work is about 100 instructions per tile for splitting P (twice that
-// for P and dS), 64 for staging, 64 for the exponentials. Two independent workgroups on a CU or wave priorities
-// did not change that. dK/dV at head dim 64 keeps K in LDS and still spills some registers.
+// 1,024 x 64, counters per SIMD: 98 thousand MFMA cycles and 93 thousand of vector issue, of 214 thousand
+// busy; no bank conflicts). Per tile and wave: about 90 vector instructions for splitting P (twice that for P and
+// dS), 130 for staging, 60 for the exponentials. Eight row tiles per workgroup halve the staging and took the
+// same time within 7%; wave priorities changed nothing. dK/dV at head dim 64 keeps K in LDS and still spills.
 //
 // Measured (us, block kernels on the float32 MFMA -> here, forward / backward; one MI355X):
 //   4 x 16 x 1,024 x 64   172 / 531 -> 111 / 352       causal  127 / 402 -> 67 / 230
