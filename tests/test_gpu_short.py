@@ -36,3 +36,45 @@ def test_short_rows_match_the_block_kernels(n, d, causal, dtype):
     want = _backward(q, k, v, o, m, do, causal, scale, config={"dkdv": 0, "dq": 0})
     for name, a, b in zip(("dq", "dk", "dv"), got, want):
         assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [16, 32, 64, 128])
+@pytest.mark.parametrize("n", NS)
+def test_short_forward_gives_the_bits_of_the_block_kernels(n, d, causal, dtype):
+    """Scores of ordinary size (N(0, 1) scaled by 1/sqrt(d)): the same max in the exponent, the same rounded
+    P and the same order of sums as the block kernels, so O and M are theirs exactly."""
+    from tattn.api import _forward
+
+    g = torch.Generator(device="cuda").manual_seed(2000 * d + n)
+    q, k, v = (torch.randn((2, 3, n, d), device="cuda", dtype=dtype, generator=g) for _ in range(3))
+    o, m = _forward(q, k, v, causal, d ** -0.5)
+    ob, mb = _forward(q, k, v, causal, d ** -0.5, config={"id": 0})
+    assert torch.equal(o, ob) and torch.equal(m, mb)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("low", [-8.0, -40.0, -3000.0, float("-inf")])
+def test_short_rows_whose_first_tile_scores_far_below_the_rest(low, causal, dtype):
+    """Keys 0-31 hidden by one component of k (left padding; its product with q is 8 low, exact in both types):
+    rows that see later keys take their max from those. O against float64: one rounding of each P and of
+    O (u relative each, |v| bounds the values)."""
+    from tattn.api import _forward
+
+    n, scale = 100, 0.125
+    g = torch.Generator(device="cuda").manual_seed(7)
+    q, k, v = (torch.randn((2, 3, n, 64), device="cuda", dtype=dtype, generator=g) for _ in range(3))
+    q[..., 0] = 8.0
+    k[..., 0] = 0.0
+    k[:, :, :32, 0] = low
+    o, m = _forward(q, k, v, causal, scale)
+    s = torch.matmul(q.double(), k.double().transpose(-1, -2).contiguous()) * scale
+    if causal:
+        s = s.masked_fill(torch.ones(n, n, dtype=torch.bool, device="cuda").triu(1), float("-inf"))
+    want = torch.matmul(torch.softmax(s, -1), v.double())
+    rows = slice(32 if causal else 0, n)  # causal: earlier rows see hidden keys only
+    u = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    assert (o.double() - want)[:, :, rows].abs().max().item() <= 3 * u * v.float().abs().max().item()
+    assert (m.double() - torch.logsumexp(s, -1) / 0.6931471805599453)[:, :, rows].abs().max().item() <= 2 * u / 0.69

@@ -8,7 +8,11 @@
 // here a slice's rows are read once, land in LDS (rows in perm32 order, chunks swizzled, as in
 // bwd_pipe.h) and everything is computed from there with one barrier.
 //
-//   forward   S^T of every key tile at once, softmax with the exact row max, O^T += V^T P^T.
+//   forward   S^T of every key tile at once, softmax, O^T += V^T P^T. The max in the exponent is
+//             the row max of tile 0, which the block kernels start from and keep at least while no score
+//             rises more than 2^kRescaleLog2 above it, and tile sums are added tile by tile: O and M
+//             are then theirs bit for bit. Rows that do rise take the max over all their keys at
+//             once, where the block kernels rescale on the way.
 //   backward  delta of the wave's queries; then, as owner of a key tile, dV and dK over the
 //             slice's query tiles; then, as owner of a query tile, dQ over its key tiles. Same
 //             operands, MFMA chains and orders as dkdv_pipe_kernel and dq_pipe_kernel, so the
@@ -143,7 +147,7 @@ __global__ __launch_bounds__(256, (fwd_short_occ<D, TT>())) void fwd_short_kerne
     const int key = 32 * t + kappa(r, h2);
     return key >= N || (CAUSAL && key > q);
   };
-  float mx = -__builtin_inff();
+  float mx = -__builtin_inff(), mx0 = mx;
 #pragma unroll
   for (int t = 0; t < TT; ++t)
     if (t < nt) {
@@ -154,14 +158,20 @@ __global__ __launch_bounds__(256, (fwd_short_occ<D, TT>())) void fwd_short_kerne
 #pragma unroll
         for (int r = 0; r < 16; ++r) mx = __builtin_fmaxf(mx, s[t][r] * c);
       }
+      if (t == 0) mx0 = mx;
     }
   mx = max_halves(mx);
+  if constexpr (TT > 1) {
+    mx0 = max_halves(mx0);
+    mx = mx > mx0 + kRescaleLog2 ? mx : mx0;
+  }
   float sum = 0.0f;
   f32x16 acc[DT];
 #pragma unroll
   for (int u = 0; u < DT; ++u) acc[u] = f32x16{};
   auto probs = [&](int t, V8 (&x)[2], auto mask_tag) {
     constexpr bool MASK = decltype(mask_tag)::value;
+    float ps = 0.0f;
 #pragma unroll
     for (int sg = 0; sg < 2; ++sg)
 #pragma unroll
@@ -174,10 +184,11 @@ __global__ __launch_bounds__(256, (fwd_short_occ<D, TT>())) void fwd_short_kerne
           if constexpr (MASK) e[b] = hidden(t, r) ? 0.0f : e[b];
         }
         const V2 pr = H::pack(e[0], e[1]);
-        sum = H::sum2(pr, sum);
+        ps = H::sum2(pr, ps);
         x[sg][i] = pr[0];
         x[sg][i + 1] = pr[1];
       }
+    sum += ps;
   };
 #pragma unroll
   for (int t = 0; t < TT; ++t)
