@@ -109,3 +109,55 @@ def test_overlapping_rows_take_the_block_kernels():
     k, v = (_rand((2, 4, 1, 64), 2 + s).expand(2, 4, 100, 64) for s in range(2))
     got, want = _forward(q, k, v, False, 0.125), _forward(q, k, v, False, 0.125, config={"id": 0})
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def _hidden_keys(shape, causal, scale, hide, low, q0):
+    """q, k, v whose keys in `hide` score q0 * low on top; the forward's O and M against float64: scores of
+    visible keys are sums of D products and rows sums of up to N, each a rounding of 2^-24, in the norm."""
+    from tattn.api import _forward
+
+    z, h, n, d = shape
+    q, k, v = (_rand(shape, 200 + s) for s in range(3))
+    q[..., 0] = q0
+    k[..., 0] = 0.0
+    k[:, :, hide, 0] = low
+    s = torch.matmul(q.double(), k.double().transpose(-1, -2).contiguous()) * scale
+    if low == -math.inf:
+        s[..., hide] = -math.inf
+    s = torch.where(s < -1e37, torch.full_like(s, -math.inf), s)  # below float32's range (or hidden by far)
+    if causal:
+        s = s.masked_fill(torch.ones(n, n, dtype=torch.bool, device="cuda").triu(1), -math.inf)
+    seen = (s > -1e6).any(-1)  # rows with a visible key
+    assert seen.float().mean() > 0.4
+    want = torch.matmul(torch.softmax(s, -1), v.double())
+    o, m = _forward(q, k, v, causal, scale)
+    assert torch.isfinite(o[seen]).all() and torch.isfinite(m[seen]).all()
+    bound = 4 * math.sqrt(n + d) * 2.0 ** -24
+    assert (o.double() - want)[seen].norm().item() <= bound * want[seen].norm().item()
+    assert (m.double() - torch.logsumexp(s, -1) / math.log(2))[seen].abs().max().item() <= 1e-6 * (1 + m[seen].abs().max().item())
+
+
+# Waves per row tile and tiles per step: {2, 4}, {4, 2}, {4, 1}, {1, 1}; head dim 128 {2, 2}, {4, 1}.
+SHAPES = [(2, 4, 128, 64), (4, 16, 512, 64), (40, 16, 512, 64), (2, 3, 30, 32), (1, 8, 600, 128), (16, 16, 600, 128)]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("low", [-1e10, -1e20, -1e30, -3.4028234663852886e38, -math.inf])
+@pytest.mark.parametrize("side", ["right", "left", "middle"])
+def test_keys_hidden_by_very_low_scores(shape, causal, low, side):
+    """Padding written into one component of k: whole tiles, so that a wave sees hidden keys first, last or only."""
+    n = shape[2]
+    edge = min(32, n // 2)
+    hide = {"right": slice(edge, n), "left": slice(0, n // 2), "middle": slice(edge, n - edge // 2)}[side]
+    _hidden_keys(shape, causal, 0.125, hide, low, 1.0)
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("causal", [False, True])
+def test_infinitely_low_scores_of_some_rows_leave_the_others(shape, causal):
+    """Even rows overflow to -inf on the hidden keys, odd rows (q = 2^-126 there) score a few below zero."""
+    n = shape[2]
+    q0 = torch.tensor([16.0, 2.0 ** -126], device="cuda").repeat((n + 1) // 2)[:n]
+    for hide in (slice(0, n // 2), slice(min(32, n // 2), n)):
+        _hidden_keys(shape, causal, 0.125, hide, -3e38, q0)

@@ -408,9 +408,8 @@ __global__ __launch_bounds__(RW * CS * 64, OCC) void fwd_f32_kernel(const FwdPar
     const float cand = max_halves(mx);
     const bool up = cand > mrow + kRescaleLog2;
     if (__builtin_amdgcn_ballot_w64(up)) {
-      const float mnew = up ? cand : mrow;
-      const float alpha = fast_exp2(mrow - mnew);
-      mrow = mnew;
+      const float alpha = up ? fast_exp2(mrow - cand) : 1.0f;  // a row that stays at -inf stays as it is
+      mrow = up ? cand : mrow;
       lrow *= alpha;
 #pragma unroll
       for (int u = 0; u < DT; ++u) acc[u] *= alpha;
@@ -418,7 +417,17 @@ __global__ __launch_bounds__(RW * CS * 64, OCC) void fwd_f32_kernel(const FwdPar
     // No key with a score above -inf so far: exponents against 0 (probability 0), not against -inf.
     const float base = mrow == -__builtin_inff() ? 0.0f : mrow;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = fast_exp2(__builtin_fmaf(s[r], c, -base));
+    for (int r = 0; r < 16; ++r) s[r] = __builtin_fmaf(s[r], c, -base);
+    // The max is a rounded product, which the FMA does not round: an exponent is at most kRescaleLog2 plus
+    // half an ulp of the max. That is below 2 up to 2^24; beyond it (keys hidden by a huge negative score,
+    // all that this wave has seen so far) it is cut, or P would be infinite and 0 times it, where a later
+    // tile or another wave raises the max, not 0.
+    if (__builtin_amdgcn_ballot_w64(__builtin_fabsf(base) > 0x1p24f)) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = s[r] > kRescaleLog2 + 2.0f ? kRescaleLog2 + 2.0f : s[r];
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = fast_exp2(s[r]);
     if (mask) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[r] = kappa(r, 0) > past ? 0.0f : s[r];
