@@ -25,6 +25,10 @@ def test_one_layout_rule():
     assert not _one_layout(a.contiguous(), off)
     wide = torch.empty_strided((1, 1, 1024, 64), (0, 0, 1 << 20, 1), dtype=torch.float16, device="meta")  # 2 GiB slices
     assert not _one_layout(wide, wide)
+    row = torch.empty(2, 3, 1, 32, dtype=torch.float16).expand(2, 3, 20, 32)  # one row, 20 times
+    assert not _one_layout(row, row)
+    window = torch.empty(2, 3, 20 * 16 + 16, dtype=torch.float16).unfold(2, 32, 16)  # rows that share halves
+    assert window.stride(2) == 16 and not _one_layout(window, window)
 
 
 @pytest.mark.gpu
@@ -56,3 +60,36 @@ def test_backward_in_place_gives_the_bits_of_copies(shape, dtype, causal, packed
     got = _backward(qv, kv, vv, ov, m, dov, causal, scale)
     for name, a, b in zip(("dq", "dk", "dv"), got, want):
         assert a.is_contiguous() and torch.equal(a, b), name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("stride", [0, 16])
+@pytest.mark.parametrize("n,d", [(1, 64), (20, 32), (100, 64), (300, 64), (513, 32), (200, 128)])
+def test_overlapping_rows(n, d, stride, dtype):
+    """All five inputs as rows that overlap (one row n times; rows 16 elements apart): rows past the end
+    of the sequence hold data there. `_backward` copies them; the library call runs its generic kernels
+    (4 waves, 32 rows per step) on them as they are. Each gives the bits of contiguous copies."""
+    from tattn import _lib
+    from tattn.api import _DTYPES, _backward, _forward
+
+    z, h, scale = 2, 3, 0.125
+    g = torch.Generator(device="cuda").manual_seed(n + d + stride)
+    span = (n - 1) * stride + d
+    views = [torch.randn(z * h * span, device="cuda", generator=g).to(dtype).as_strided((z, h, n, d), (h * span, span, stride, 1))
+             for _ in range(5)]
+    copies = [t.contiguous().clone() for t in views]
+    _, m = _forward(copies[0], copies[1], copies[2], False, scale)
+    want = _backward(copies[0], copies[1], copies[2], copies[3], m, copies[4], False, scale)
+    got = _backward(views[0], views[1], views[2], views[3], m, views[4], False, scale)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    grads = [torch.empty_like(copies[0]) for _ in range(3)]
+    delta = torch.empty_like(m)
+    rc = _lib.load().tattn_bwd_layouts(*(t.data_ptr() for t in (*views, *grads, m, delta)), _lib.strides4(views[0]),
+                                       _lib.strides4(copies[0]), z, h, n, d, _DTYPES[dtype], 0, scale, -1,
+                                       torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    generic = {"dkdv": {"kind": 0, "block_n": 128, "block_m": 32}, "dq": {"kind": 0, "block_m": 128, "block_n": 32}}
+    want = _backward(copies[0], copies[1], copies[2], copies[3], m, copies[4], False, scale, config=generic)
+    for name, a, b in zip(("dq", "dk", "dv"), grads, want):
+        assert torch.equal(a, b), name

@@ -516,7 +516,7 @@ int tattn_bwd_layouts(const void* q, const void* k, const void* v, const void* o
                         Z, H, N, D, dtype, causal, sm_scale, config_id)))
     return rc;
   const hipStream_t st = (hipStream_t)stream;
-  if (config_id < 0 && bwd_short_fits(p, dtype)) return launch_bwd_short(p, (int)D, dtype, causal != 0, st);
+  if (config_id < 0 && bwd_short_fits(p, (int)D, dtype)) return launch_bwd_short(p, (int)D, dtype, causal != 0, st);
   if (fuse) {
     BwdParams pq = p;
     pq.fuse_delta = 1;

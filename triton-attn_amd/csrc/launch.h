@@ -45,10 +45,13 @@ int launch_dkdv_persist(const BwdParams& p, int D, int dtype, int config_id, boo
 // p.n_blocks set by the caller; the caller has checked bwd_fits32.
 int launch_split(const BwdParams& p, int D, int dtype, bool dkdv, bool causal, hipStream_t st);
 
-// Whether the backward's (z, h) slices fit 32-bit buffer offsets (plus two steps of look-ahead):
-// the pipelined and persistent backward kernels need it, the generic ones take 64-bit addresses.
+// Whether the backward's (z, h) slices fit 32-bit buffer offsets (plus two steps of look-ahead) and
+// rows past the sequence end lie past the slice's last byte, so that range-checked loads give zeros for
+// them (rows that overlap, such as a broadcast row of stride 0, do not: queries past the end would add
+// to dK and dV). Every backward kernel but the generic ones needs both; those check row indices and take
+// 64-bit addresses.
 inline bool bwd_fits32(const BwdParams& p, int D) {
-  return slice_bytes(p.N, p.s[2], D) + (uint64_t)p.s[2] * 128 < (1ull << 31);
+  return p.s[2] >= D && slice_bytes(p.N, p.s[2], D) + (uint64_t)p.s[2] * 128 < (1ull << 31);
 }
 
 // Short rows (short.hip): up to 128 rows of a slice in one workgroup's waves, the whole backward in
@@ -60,8 +63,8 @@ int launch_bwd_short(const BwdParams& p, int D, int dtype, bool causal, hipStrea
 inline bool fwd_short_fits(const FwdParams& p, int dtype) {
   return dtype != 1 && p.N <= kShortRows && (p.sk[2] | p.sv[2]) * 256 < (1ll << 30);
 }
-inline bool bwd_short_fits(const BwdParams& p, int dtype) {
-  return dtype != 1 && p.N <= kShortRows && p.s[2] * 256 < (1ll << 30);
+inline bool bwd_short_fits(const BwdParams& p, int D, int dtype) {
+  return dtype != 1 && p.N <= kShortRows && p.s[2] >= D && p.s[2] * 256 < (1ll << 30);
 }
 
 // Waves of a workgroup split the summed dimension (coop.hip); 16-bit, slices that fit 32-bit

@@ -103,8 +103,8 @@ def _kernel_layout(t: torch.Tensor) -> torch.Tensor:
 
 def _one_layout(q: torch.Tensor, *others: torch.Tensor) -> bool:
     """Whether the backward reads these tensors where they lie: one (z, h, n) layout for all of
-    them that the kernels take (`_kernel_layout`), with slices that 32-bit offsets span (beyond
-    that the kernels for wide slices are slower than a contiguous copy). Token-major activations,
+    them that the kernels take (`_kernel_layout`), with rows that do not overlap and slices that
+    32-bit offsets span (the kernels for other layouts are slower than a contiguous copy). Token-major activations,
     the output that inherits their layout and its gradient are the usual case; the five copies
     that the reference's backward starts with (api.py:111) took 78 us of 334 at 11 x 12 x 1500
     tokens x 64 in fp16, forward + backward, and 106 us of 721 at 2 x 16 x 4096 x 128 in bf16."""
@@ -119,6 +119,7 @@ def _one_layout(q: torch.Tensor, *others: torch.Tensor) -> bool:
         ptrs % 16 == 0
         and st[3] == 1
         and (st[0] * size) % 16 == 0 and (st[1] * size) % 16 == 0 and (st[2] * size) % 16 == 0
+        and st[2] >= q.shape[3]
         and (q.shape[2] + 127) * st[2] * size < 1 << 31
     )
 
