@@ -2,13 +2,15 @@
 // with float32 inputs): every float32 operand as an exact sum of three bf16 planes.
 //
 // The float32 MFMA runs at 1/16 of the bf16 rate and bounds the kernels built on it. Here x = hi + mid +
-// lo (hi: the top 8 significant bits, mid and lo the roundings of what is left: all 24 bits are held),
-// and a product of two operands is the six bf16 products of plane pairs down to 2^-16 of it, smallest
-// first, into a float32 accumulator; what is dropped (mid lo, lo mid, lo lo) is below 2^-21 of a
-// product. Probabilities and dS are split the same way, so nothing is held in 16 bits. A bf16 MFMA adds
-// 16 products per rounding of the accumulator where the float32 one adds 2: the error against float64
-// is below the float32 MFMA kernels' at every size measured (relative, O / dK: 4 x 16 x 1,024 x 64 5.4e-7 / 6.7e-7
-// against 6.4e-7 / 7.5e-7; 1 x 4 x 4,096 x 64 causal 2.7e-7 / 7.0e-7 against 5.0e-7 / 1.6e-6).
+// lo (all 24 bits are held), and a product of two operands is the six bf16 products of plane pairs down to
+// 2^-16 of it, smallest first, into a float32 accumulator. What is dropped (mid lo, lo mid, lo lo) is at
+// most 2^-24.1 of a product of two inputs, 2^-27.4 in the root mean square, and 2^-23.3 and 2^-26.4 for P and dS
+// times an input (4 million pairs each; a float32 product's rounding is 2^-24.0 and 2^-25.2). P and dS are split
+// the same way, so nothing is held in 16 bits. A bf16 MFMA adds 16 products per rounding of the accumulator
+// where the float32 one adds 2: the error against float64 is below the float32 MFMA kernels' at every size
+// from N = 4 to 4,096 and every head dim (relative, O / dK: 1,024 slices x 16 x 16
+// 8.2e-8 / 1.7e-7 against 1.3e-7 / 2.1e-7; 8 x 1,024 x 64 3.3e-7 / 4.7e-7 against 6.5e-7 / 7.5e-7; 4 x 4,096 x 64 causal
+// 2.7e-7 / 6.9e-7 against 5.0e-7 / 1.5e-6).
 //
 // A bf16 plane cannot carry what an infinite float32 operand means (inf - inf has no middle plane) nor
 // all bits of numbers near the smallest exponents. Where a wave's operands hold an infinity, or are all
@@ -27,11 +29,10 @@
 // same time within 7%; wave priorities changed nothing. dK/dV at head dim 64 keeps K in LDS and still spills.
 //
 // Measured (us, block kernels on the float32 MFMA -> here, forward / backward; one MI355X):
-//   4 x 16 x 1,024 x 64   172 / 531 -> 111 / 352       causal  127 / 402 -> 67 / 230
-//   2 x 4 x 128 x 64      18.3 / 57 -> 10.1 / 36        1 x 4 x 4,096 x 64 causal  371 / 1,144 -> 118 / 407
-//   2 x 16 x 2,048 x 128  792 / 2,177 -> 500 / 2,109    2 x 8 x 1,000 x 128 causal  184 / 575 -> 94 / 369
-//   8 x 16 x 512 x 32     51 / 157 -> 37 / 101          3 x 5 x 777 x 16  46 / 123 -> 18 / 45
-#include <cfloat>
+//   4 x 16 x 1,024 x 64   172 / 531 -> 110 / 341       causal  127 / 402 -> 65 / 227
+//   2 x 4 x 128 x 64      18.3 / 57 -> 10.1 / 39        1 x 4 x 4,096 x 64 causal  371 / 1,144 -> 119 / 403
+//   2 x 16 x 2,048 x 128  792 / 2,177 -> 515 / 2,089    2 x 8 x 1,000 x 128 causal  184 / 575 -> 92 / 342
+//   8 x 16 x 512 x 32     51 / 157 -> 37 / 98           3 x 5 x 777 x 16  46 / 123 -> 16 / 41
 #include <type_traits>
 
 #include "bwd_pipe.h"
@@ -56,21 +57,28 @@ __device__ __forceinline__ bf16x2 tops(float a, float b) {  // upper halves of a
   return __builtin_bit_cast(bf16x2, __builtin_amdgcn_perm(bits(b), bits(a), 0x07060302u));
 }
 
-// hi truncated (cannot overflow), mid and lo rounded to nearest (lo exactly representable).
+// mid and lo rounded to nearest (lo exactly representable). hi: the nearest bf16 (ties away from zero) for
+// operands that are LOADED, own rows and staged rows alike, so that S has the same bits in every kernel;
+// truncated for those made in registers, which need no rounded copy then (with it the backward spills 16
+// registers more: 4 x 16 x 1,024 x 64 345 -> 387 us). The rounding is an integer add (with v_cvt_pk dK/dV at head
+// dim 64 takes 4 us more per launch: 256 x 128 rows 30.2 -> 34.4, against 30.3 with the add).
+template <bool LOADED>
 __device__ __forceinline__ void split2(float a, float b, bf16x2& hi, bf16x2& mid, bf16x2& lo) {
-  hi = tops(a, b);
-  const float ra = a - top(a), rb = b - top(b);
+  const float ha = LOADED ? __builtin_bit_cast(float, bits(a) + 0x8000u) : a;
+  const float hb = LOADED ? __builtin_bit_cast(float, bits(b) + 0x8000u) : b;
+  hi = tops(ha, hb);
+  const float ra = a - top(ha), rb = b - top(hb);
   mid = H::pack(ra, rb);
   const uint32_t m = __builtin_bit_cast(uint32_t, mid);
   lo = H::pack(ra - __builtin_bit_cast(float, m << 16), rb - __builtin_bit_cast(float, m & 0xffff0000u));
 }
-template <typename F>
+template <bool LOADED = false, typename F>
 __device__ __forceinline__ Planes split8(F at) {
   Planes p;
 #pragma unroll
   for (int i = 0; i < 8; i += 2) {
     bf16x2 h, m, l;
-    split2(at(i), at(i + 1), h, m, l);
+    split2<LOADED>(at(i), at(i + 1), h, m, l);
     p.hi[i] = h[0], p.hi[i + 1] = h[1];
     p.mid[i] = m[0], p.mid[i + 1] = m[1];
     p.lo[i] = l[0], p.lo[i + 1] = l[1];
@@ -130,10 +138,11 @@ __device__ __forceinline__ f32x16 mm32(const Planes& a, bool raw, F b, f32x16 c)
 }
 
 // Whether a wave's operand values (the lane's largest magnitude, not-a-numbers aside) need the float32
-// MFMA: an infinity, or nothing but numbers so small that their planes would lose bits.
-constexpr float kSmall = 0x1p-40f;
+// MFMA: an infinity or a number that bf16 rounds to one, or nothing but numbers so small that their planes
+// would lose bits.
+constexpr float kLarge = 0x1.ffp127f, kSmall = 0x1p-40f;
 __device__ __forceinline__ bool needs32(float amax) {
-  return __builtin_amdgcn_ballot_w64(amax > FLT_MAX) != 0 ||
+  return __builtin_amdgcn_ballot_w64(amax >= kLarge) != 0 ||
          (__builtin_amdgcn_ballot_w64(amax >= kSmall) == 0 && __builtin_amdgcn_ballot_w64(amax > 0.0f) != 0);
 }
 
@@ -194,8 +203,8 @@ struct Stager {
     for (int i = 0; i < S::PW; ++i) {
       if (!live(i)) continue;
       bf16x2 h[2], m[2], l[2];
-      split2(x[i][0], x[i][1], h[0], m[0], l[0]);
-      split2(x[i][2], x[i][3], h[1], m[1], l[1]);
+      split2<true>(x[i][0], x[i][1], h[0], m[0], l[0]);
+      split2<true>(x[i][2], x[i][3], h[1], m[1], l[1]);
       TATTN_LDS char* d = (TATTN_LDS char*)stage + dst[i];
       *reinterpret_cast<TATTN_LDS bf16x4*>(d) = bf16x4{h[0][0], h[0][1], h[1][0], h[1][1]};
       *reinterpret_cast<TATTN_LDS bf16x4*>(d + S::TILE) = bf16x4{m[0][0], m[0][1], m[1][0], m[1][1]};
@@ -289,7 +298,7 @@ struct OwnRows {
     each([&](int s, f32x4 a, f32x4 b) __attribute__((always_inline)) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) amax = __builtin_fmaxf(amax, __builtin_fmaxf(__builtin_fabsf(a[i]), __builtin_fabsf(b[i])));
-      set(s, split8([&](int i) { return i < 4 ? a[i & 3] : b[i & 3]; }));
+      set(s, split8<true>([&](int i) { return i < 4 ? a[i & 3] : b[i & 3]; }));
     });
     return needs32(amax);
   }
@@ -511,12 +520,12 @@ __global__ __launch_bounds__(RW * CS * 64, OCC) void fwd_f32_kernel(const FwdPar
   }
 }
 
-// Largest magnitude of a tile's probabilities and dS (the MFMA operands made in registers) is finite.
+// Largest magnitude of a tile's probabilities and dS (the MFMA operands made in registers) is finite in bf16.
 __device__ __forceinline__ bool all_finite(const f32x16& a) {
   float m = 0.0f;
 #pragma unroll
   for (int r = 0; r < 16; ++r) m = __builtin_fmaxf(m, __builtin_fabsf(a[r]));
-  return __builtin_amdgcn_ballot_w64(m > FLT_MAX) == 0;
+  return __builtin_amdgcn_ballot_w64(m >= kLarge) == 0;
 }
 
 // ---- dQ --------------------------------------------------------------------------------------

@@ -81,8 +81,9 @@ inline bool bwd_coop_fits(const BwdParams& p, int D, int dtype) {
 }
 
 // float32 on split operands (f32_split.hip): row offsets of a slice, with a step's look-ahead, fit 32
-// bits, and rows past the end of a slice lie past its last element (rows that overlap do not). One
-// key alone stays with the block kernels, whose O and dV are V and dO to the bit there; so do short rows at
+// bits, and rows past the end of a slice lie past its last element (rows that overlap do not). One to three
+// keys stay with the block kernels: sums of so few products are no closer to float64 here (dV of 2 keys,
+// causal, head dim 16: 5.4e-8 against 5.1e-8). So do short rows at
 // head dim 128, where one wave per SIMD is all that fits (us, forward / backward, split against block kernels:
 // 64 x 16 x 24: 41 / 159, 37 / 113; 64 x 8 x 64: 35 / 131, 37 / 119; 16 x 16 x 128 causal: 31 / 108, 40 / 122). Both
 // directions go the same way: M belongs to the bits of the forward's S.
@@ -90,7 +91,7 @@ int launch_fwd_f32(const FwdParams& p, int D, bool causal, hipStream_t st);
 int launch_dq_f32(const BwdParams& p, int D, bool causal, hipStream_t st);
 int launch_dkdv_f32(const BwdParams& p, int D, bool causal, hipStream_t st);
 inline bool f32_rows_fit(int64_t N, int64_t row_stride, int D) {
-  return N > (D < 128 ? 1 : 96) && row_stride >= D && row_stride < (1ll << 22) && (N + 256) * row_stride * 4 < (1ll << 31);
+  return N > (D < 128 ? 3 : 96) && row_stride >= D && row_stride < (1ll << 22) && (N + 256) * row_stride * 4 < (1ll << 31);
 }
 inline bool fwd_f32_fits(const FwdParams& p, int D) { return f32_rows_fit(p.N, p.sk[2], D) && f32_rows_fit(p.N, p.sv[2], D); }
 inline bool bwd_f32_fits(const BwdParams& p, int D) { return f32_rows_fit(p.N, p.s[2], D); }
