@@ -194,3 +194,32 @@ def test_numbers_beyond_the_largest_bf16(which):
         ok = torch.isfinite(b) & (r.abs() < 3e38)
         ea, eb, size = ((a.double() - r)[ok].norm().item(), (b.double() - r)[ok].norm().item(), r[ok].norm().item())
         assert ea <= 1.25 * eb + 2.0 ** -24 * size, (name, ea / size, eb / size)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("mag", [(1.0, 1.0, 1.0, 1e-13), (1.0, 1.0, 1.0, 1e-25), (1.0, 1.0, 1e-14, 1e-14), (1.0, 1.0, 1e-17, 1e-18),
+                                 (1e-20, 1e20, 1e-28, 1.0), (1.0, 1.0, 1e-15, 3e-21)])
+def test_small_magnitudes(mag, d, causal):
+    """Loss gradients of ordinary and of very small size (dS down to 1e-38, where planes lose bits)."""
+    _compare(*(_rand((2, 4, 150, d), 500 + s) * x for s, x in enumerate(mag)), causal, d ** -0.5)
+
+
+def test_tiny_rows_beside_ordinary_ones():
+    """Every fourth row of dO at 2^e of the others: the others keep what the block kernels give. The dS of a tiny
+    row are about 2^e * 8 / 150 (dP of 64 products, P of 150 keys), or 2^(e - 4.2), and held to 2^-134: its dQ has a
+    relative error of at most 2^(-129 - e), or that of float32 sums (2^-21)."""
+    q, k, v, do = (_rand((2, 4, 150, 64), 600 + s) for s in range(4))
+    ordinary = torch.arange(150, device="cuda") % 4 != 0
+    for e in (-95, -105, -115, -125):
+        rel = max(2.0 ** -21, 2.0 ** (-129 - e))
+        w = torch.where(ordinary, 1.0, 2.0 ** e)[:, None]
+        t = (q, k, v, do * w)
+        ref = _exact(*t, False, 0.125)
+        got, _ = _run(*t, False, 0.125, False)
+        old, _ = _run(*t, False, 0.125, True)
+        for name, a, b, r in zip(("o", "dq", "dk", "dv"), got, old, ref):
+            ea, eb = ((x.double() - r)[:, :, ordinary].norm().item() for x in (a, b))
+            assert ea <= 1.25 * eb + 2.0 ** -24 * r.norm().item(), (e, name)
+        tiny = ref[1][:, :, ~ordinary]
+        assert (got[1].double()[:, :, ~ordinary] - tiny).norm().item() <= rel * tiny.norm().item(), e

@@ -12,10 +12,11 @@
 // 8.2e-8 / 1.7e-7 against 1.3e-7 / 2.1e-7; 8 x 1,024 x 64 3.3e-7 / 4.7e-7 against 6.5e-7 / 7.5e-7; 4 x 4,096 x 64 causal
 // 2.7e-7 / 6.9e-7 against 5.0e-7 / 1.5e-6).
 //
-// A bf16 plane cannot carry what an infinite float32 operand means (inf - inf has no middle plane) nor
-// all bits of numbers near the smallest exponents. Where a wave's operands hold an infinity, or are all
-// below 2^-40 without being zero, the step is staged again as the halves of the float32 bits and runs on the
-// float32 MFMA: what the block kernels give there, at about their speed.
+// A bf16 plane cannot carry what an infinite float32 operand means (inf - inf has no middle plane), nor
+// bits below 2^-133, which numbers from 2^-110 up do not have. Where a wave's operands hold an infinity, or are all
+// below 2^-100 without being zero, the step is staged again as the halves of the float32 bits and runs on the
+// float32 MFMA: what the block kernels give there, in 1.1 to 1.5 times their time. A number below 2^-110 beside one
+// of 2^-100 or more in the same wave is held to 2^-134.
 //
 // Split of the work: a workgroup of NW = RW * CS waves owns RW 32-row tiles; a step stages CS tile
 // pairs of the other dimension (read from HBM once per workgroup, split into planes once, by the thread
@@ -86,7 +87,7 @@ __device__ __forceinline__ Planes split8(F at) {
   return p;
 }
 // The float32 value again, for the float32 MFMA: raw planes hold the two halves of its bits (lo is not
-// used), split ones its parts (exact for operands that needs32 lets pass).
+// used), split ones its parts (exact from 2^-110 up).
 __device__ __forceinline__ float whole(const Planes& p, int i, bool raw) {
   typedef uint16_t U8 __attribute__((ext_vector_type(8)));
   const U8 h = __builtin_bit_cast(U8, p.hi), m = __builtin_bit_cast(U8, p.mid);
@@ -139,8 +140,9 @@ __device__ __forceinline__ f32x16 mm32(const Planes& a, bool raw, F b, f32x16 c)
 
 // Whether a wave's operand values (the lane's largest magnitude, not-a-numbers aside) need the float32
 // MFMA: an infinity or a number that bf16 rounds to one, or nothing but numbers so small that their planes
-// would lose bits.
-constexpr float kLarge = 0x1.ffp127f, kSmall = 0x1p-40f;
+// may lose bits. (Gradients of a mean over many elements are ordinary down to 2^-60 or so: with the line at
+// 2^-40 the backward of 4 x 16 x 1,024 x 64 took 675 us on them, the block kernels 531, the planes 341.)
+constexpr float kLarge = 0x1.ffp127f, kSmall = 0x1p-100f;
 __device__ __forceinline__ bool needs32(float amax) {
   return __builtin_amdgcn_ballot_w64(amax >= kLarge) != 0 ||
          (__builtin_amdgcn_ballot_w64(amax >= kSmall) == 0 && __builtin_amdgcn_ballot_w64(amax > 0.0f) != 0);
@@ -520,12 +522,12 @@ __global__ __launch_bounds__(RW * CS * 64, OCC) void fwd_f32_kernel(const FwdPar
   }
 }
 
-// Largest magnitude of a tile's probabilities and dS (the MFMA operands made in registers) is finite in bf16.
-__device__ __forceinline__ bool all_finite(const f32x16& a) {
+// Whether the planes hold a tile's probabilities or dS (the MFMA operands made in registers).
+__device__ __forceinline__ bool planes_hold(const f32x16& a) {
   float m = 0.0f;
 #pragma unroll
   for (int r = 0; r < 16; ++r) m = __builtin_fmaxf(m, __builtin_fabsf(a[r]));
-  return __builtin_amdgcn_ballot_w64(m >= kLarge) == 0;
+  return !needs32(m);
 }
 
 // ---- dQ --------------------------------------------------------------------------------------
@@ -619,7 +621,7 @@ __global__ __launch_bounds__(RW * CS * 64, OCC) void dq_f32_kernel(const BwdPara
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] *= dp[r] - dl;
-    if (!slow && all_finite(s)) {
+    if (!slow && planes_hold(s)) {
 #pragma unroll
       for (int sl = 0; sl < 2; ++sl) {
         const Planes x = split8([&](int e) { return s[8 * sl + e]; });
@@ -765,7 +767,7 @@ __global__ __launch_bounds__(RW * CS * 64, OCC) void dkdv_f32_kernel(const BwdPa
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) dp[r] *= s[r];
-    if (!slow && all_finite(s) && all_finite(dp)) {
+    if (!slow && planes_hold(s) && planes_hold(dp)) {
 #pragma unroll
       for (int sl = 0; sl < 2; ++sl) {
         const Planes x = split8([&](int e) { return s[8 * sl + e]; });
