@@ -262,7 +262,7 @@ def backward_roofline(data, causal_modes=(False, True), reps: int = 10) -> dict:
             row = {"seq": n, "batch": b, "causal": causal}
             for name, ms, work, kern in (("dkdv", t_kv, 2.0 * f, _lib.K_BWD_DKDV), ("dq", t_q, 1.5 * f, _lib.K_BWD_DQ)):
                 tf = work / (ms * 1e-3) / 1e12
-                row[name] = {"entry": _lib.pick_config(kern, DIM, _lib.F16, causal, n), "us": round(1e3 * ms, 2),
+                row[name] = {"entry": _lib.picked(kern, (b, HEADS, n, DIM), _lib.F16, causal), "us": round(1e3 * ms, 2),
                              "exec_tflops": round(tf, 1), "frac": round(tf / PEAK_F16_TFLOPS, 4)}
             counted = 2.5 * f / (t_all * 1e-3) / 1e12
             row["tattn_bwd"] = {"us": round(1e3 * t_all, 2), "counted_tflops": round(counted, 1),
@@ -410,7 +410,10 @@ def main() -> int:
     from tattn import _lib
 
     def entry_name(n: int) -> str:
-        cfg = _lib.config_desc(_lib.K_FWD, DIM, _lib.F16, _lib.pick_config(_lib.K_FWD, DIM, _lib.F16, a.causal, n))
+        pick = _lib.picked(_lib.K_FWD, (data[n][0], HEADS, n, DIM), _lib.F16, a.causal)
+        if pick in _lib.PICK_NAMES:
+            return f"fwd_{_lib.PICK_NAMES[pick]}_kernel"
+        cfg = _lib.config_desc(_lib.K_FWD, DIM, _lib.F16, pick)
         kind = {2: f"fwd_persist_kernel, ring {cfg['ring']}", 1: "fwd_pipe_kernel"}.get(cfg["kind"], "fwd_generic_kernel")
         return f"{kind}, {cfg['waves']} waves x {cfg['tiles']} tiles ({cfg['block_m']} query rows per workgroup)"
 

@@ -143,14 +143,30 @@ int tattn_bwd_noalloc(const void* q, const void* k, const void* v, const void* o
 /*
  * Tile table introspection (the gfx950 replacement of the reference's autotune config lists,
  * src/tattn/kernels.py:21-54): number of entries for (kernel, D, dtype), the entry itself, and
- * the entry the library picks for a problem (the reference keys its autotuner on
- * (N bucket, head dim, causal), kernels.py:57-61 and api.py:59-62). tattn_pick_config reports
- * the pick for a batch x heads count that is a multiple of 8; the entry points also take the
- * batch x heads count into account (the persistent forward needs whole slices per XCD).
+ * the table entry ranked first for a launch that fills the GPU with a batch x heads count that is a
+ * multiple of 8 (the reference keys its autotuner on (N bucket, head dim, causal), kernels.py:57-61
+ * and api.py:59-62). What a call with config_id -1 runs depends on the whole problem and may be a
+ * kernel outside the table: tattn_picked.
  */
 int tattn_num_configs(int kernel, int64_t D, int dtype);
 int tattn_config_desc(int kernel, int64_t D, int dtype, int config_id, tattn_config* out);
 int tattn_pick_config(int kernel, int64_t D, int dtype, int causal, int64_t N);
+
+/* Kernels outside the table, as tattn_picked reports them. */
+enum tattn_pick {
+  TATTN_PICK_COOP = 1000,   /* 16-bit, few rows: the waves of a workgroup split the summed dimension */
+  TATTN_PICK_PLANES = 1001, /* float32 on the 16-bit matrix cores, operands as three planes */
+  TATTN_PICK_SHORT = 1002   /* 16-bit, N <= 128: whole slices in LDS, the whole backward in one launch */
+};
+
+/*
+ * What a call with config_id -1 runs for a problem: a table index or a tattn_pick. Forward
+ * (TATTN_K_FWD): strides of k and of v. Backward kernels, as tattn_bwd and its variants run them:
+ * k_strides are the strides the inputs share, v_strides is not read. Null strides: contiguous
+ * (v_strides: those of k). -1 for arguments the entry points refuse. Launches nothing.
+ */
+int tattn_picked(int kernel, const int64_t k_strides[4], const int64_t v_strides[4], int64_t Z, int64_t H,
+                 int64_t N, int64_t D, int dtype, int causal, float sm_scale);
 
 #ifdef __cplusplus
 }

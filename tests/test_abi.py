@@ -150,3 +150,31 @@ def test_picks_at_the_benchmark_lengths(n, dtype):
             assert dkdv64["kind"] == 1 and dkdv64["waves"] == 8
         assert dq64["kind"] == 2 and dq64["waves"] == 4
         assert kind(_lib.K_BWD_DKDV, 128, causal)["kind"] == 3 and kind(_lib.K_BWD_DQ, 128, causal)["kind"] == 3
+
+
+@pytest.mark.parametrize("kernel", [_lib.K_FWD, _lib.K_BWD_DKDV, _lib.K_BWD_DQ])
+def test_picked_names_the_kernel_that_a_call_runs(kernel):
+    """tattn_picked: kernels outside the tables for short rows, few rows and float32 where their
+    preconditions hold, table entries elsewhere."""
+    def pick(shape, dtype, causal=True, **kw):
+        return _lib.picked(kernel, shape, dtype, causal, **kw)
+
+    for dtype in (_lib.F16, _lib.BF16):
+        for n in (1, 32, 128):
+            assert pick((2, 8, n, 64), dtype) == _lib.PICK_SHORT
+        assert pick((1, 16, 2048, 64), dtype) == _lib.PICK_COOP
+        assert 0 <= pick((64, 16, 2048, 64), dtype) < _lib.num_configs(kernel, 64, dtype)
+        # Rows 16 MiB apart: beyond the 32-bit offsets of all kernels but the generic ones.
+        assert pick((1, 16, 2048, 64), dtype, strides=(0, 64, 1 << 23, 1)) < _lib.num_configs(kernel, 64, dtype)
+    if kernel == _lib.K_FWD:  # hides keys at a score of -inf, which scale 0 does not have
+        assert pick((1, 16, 2048, 64), _lib.F16, scale=0.0) < _lib.num_configs(kernel, 64, _lib.F16)
+    else:  # rows that overlap
+        assert pick((2, 8, 100, 64), _lib.F16, strides=(64, 64, 0, 1)) < _lib.num_configs(kernel, 64, _lib.F16)
+    assert pick((4, 16, 1024, 64), _lib.F32) == _lib.PICK_PLANES
+    for shape in ((4, 16, 3, 64), (4, 16, 96, 128)):
+        assert pick(shape, _lib.F32) == 0
+    assert pick((4, 16, 1024, 64), _lib.F32, strides=(64, 64, 0, 1)) == 0
+    with pytest.raises(RuntimeError, match="head dim"):
+        pick((1, 1, 16, 48), _lib.F16)
+    with pytest.raises(RuntimeError, match="no kernel"):
+        _lib.picked(7, (1, 1, 16, 64), _lib.F16, False)

@@ -124,10 +124,9 @@ struct Cheapest {
   }
 };
 
-// The kernels whose waves split the summed dimension (coop.hip), as a candidate.
-constexpr int kCoop = 1000;
-// The float32 kernels on split operands (f32_split.hip).
-constexpr int kSplit = 1001;
+// Kernels outside the tables: waves that split the summed dimension (coop.hip), float32 on split operands
+// (f32_split.hip), short rows (short.hip).
+constexpr int kCoop = TATTN_PICK_COOP, kSplit = TATTN_PICK_PLANES, kShort = TATTN_PICK_SHORT;
 
 // Table pick for a problem (index into the kernel's table, or kCoop / kSplit where `own` says that
 // the problem meets the preconditions of coop.hip in 16 bits, of f32_split.hip in float32), keyed
@@ -300,6 +299,7 @@ int check_shape(int64_t Z, int64_t H, int64_t N, int64_t D, int dtype) {
 }
 
 int run_fwd(const FwdParams& p, int D, int dtype, bool causal, int id, hipStream_t st) {
+  if (id == kShort) return launch_fwd_short(p, D, dtype, causal, st);
   if (id == kSplit) return launch_fwd_f32(p, D, causal, st);
   return id == kCoop ? launch_fwd_coop(p, D, dtype, causal, st) : launch_fwd(p, D, dtype, causal, id, st);
 }
@@ -315,16 +315,20 @@ int run_dkdv(const BwdParams& p, int D, int dtype, bool causal, int id, hipStrea
 bool fwd_own_fits(const FwdParams& p, int D, int dtype) { return dtype == TATTN_F32 ? fwd_f32_fits(p, D) : fwd_coop_fits(p, D, dtype); }
 bool bwd_own_fits(const BwdParams& p, int D, int dtype) { return dtype == TATTN_F32 ? bwd_f32_fits(p, D) : bwd_coop_fits(p, D, dtype); }
 
-// A caller's table index, or the pick (own: see pick_config).
-int resolve(int kernel, int64_t D, int dtype, int causal, int64_t N, int64_t ZH, int id, bool own, int* out) {
+// What the library picks: the forward, and one kernel of the backward (the whole backward of short rows
+// is one launch: the callers that run both kernels look at bwd_short_fits first).
+int pick_fwd(const FwdParams& p, int D, int dtype, int causal) {
+  if (fwd_short_fits(p, dtype)) return kShort;
+  return pick_config(TATTN_K_FWD, D, dtype, causal, p.N, (int64_t)p.Z * p.H, fwd_own_fits(p, D, dtype));
+}
+int pick_bwd(int kernel, const BwdParams& p, int D, int dtype, int causal) {
+  return pick_config(kernel, D, dtype, causal, p.N, (int64_t)p.Z * p.H, bwd_own_fits(p, D, dtype));
+}
+
+// Whether a caller's table index exists.
+int check_config(int kernel, int64_t D, int dtype, int id) {
   const int n = num_configs(kernel, D, dtype);
-  if (id < 0) {
-    *out = pick_config(kernel, D, dtype, causal, N, ZH, own);
-    return TATTN_OK;
-  }
-  if (id >= n) return set_error(TATTN_E_CONFIG, "config id %d out of range [0, %d)", id, n);
-  *out = id;
-  return TATTN_OK;
+  return id < n ? TATTN_OK : set_error(TATTN_E_CONFIG, "config id %d out of range [0, %d)", id, n);
 }
 
 }  // namespace
@@ -369,6 +373,26 @@ int tattn_pick_config(int kernel, int64_t D, int dtype, int causal, int64_t N) {
   return pick_config(kernel, D, dtype, causal, N, 1 << 16, false);  // a full chip, Z * H a multiple of 8
 }
 
+int tattn_picked(int kernel, const int64_t k_strides[4], const int64_t v_strides[4], int64_t Z, int64_t H, int64_t N,
+                 int64_t D, int dtype, int causal, float sm_scale) {
+  if (check_shape(Z, H, N, D, dtype)) return -1;
+  const int64_t whole[4] = {H * N * D, N * D, D, 1};
+  if (!k_strides) k_strides = whole;
+  if (!v_strides) v_strides = k_strides;
+  if (kernel == TATTN_K_FWD) {
+    FwdParams p{};
+    for (int i = 0; i < 3; ++i) p.sk[i] = k_strides[i], p.sv[i] = v_strides[i];
+    p.Z = (int32_t)Z; p.H = (int32_t)H; p.N = (int32_t)N;
+    p.c = sm_scale * kLog2e;
+    return pick_fwd(p, (int)D, dtype, causal);
+  }
+  if (kernel != TATTN_K_BWD_DKDV && kernel != TATTN_K_BWD_DQ) return set_error(TATTN_E_ARG, "no kernel %d", kernel), -1;
+  BwdParams p{};
+  for (int i = 0; i < 3; ++i) p.s[i] = k_strides[i];
+  p.Z = (int32_t)Z; p.H = (int32_t)H; p.N = (int32_t)N;
+  return bwd_short_fits(p, (int)D, dtype) ? kShort : pick_bwd(kernel, p, (int)D, dtype, causal);
+}
+
 int tattn_fwd(const void* q, const void* k, const void* v, void* o, float* m, const int64_t q_strides[4],
               const int64_t k_strides[4], const int64_t v_strides[4], const int64_t o_strides[4], int64_t Z,
               int64_t H, int64_t N, int64_t D, int dtype, int causal, float sm_scale, int config_id,
@@ -387,10 +411,8 @@ int tattn_fwd(const void* q, const void* k, const void* v, void* o, float* m, co
   }
   p.Z = (int32_t)Z; p.H = (int32_t)H; p.N = (int32_t)N;
   p.c = sm_scale * kLog2e;
-  int id;
-  if ((rc = resolve(TATTN_K_FWD, D, dtype, causal, N, Z * H, config_id, fwd_own_fits(p, (int)D, dtype), &id))) return rc;
-  if ((rc = device_check())) return rc;
-  if (config_id < 0 && fwd_short_fits(p, dtype)) return launch_fwd_short(p, (int)D, dtype, causal != 0, (hipStream_t)stream);
+  if ((rc = check_config(TATTN_K_FWD, D, dtype, config_id)) || (rc = device_check())) return rc;
+  const int id = config_id < 0 ? pick_fwd(p, (int)D, dtype, causal) : config_id;
   return run_fwd(p, (int)D, dtype, causal != 0, id, (hipStream_t)stream);
 }
 
@@ -431,9 +453,8 @@ int tattn_bwd_dkdv(const void* q, const void* k, const void* v, const void* dout
       (rc = check_tensor("dk", dk, strides, sz)) || (rc = check_tensor("dv", dv, strides, sz)))
     return rc;
   if (!m || !delta) return set_error(TATTN_E_ARG, "m and delta must not be null");
-  int id;
-  if ((rc = resolve(TATTN_K_BWD_DKDV, D, dtype, causal, N, Z * H, config_id, bwd_own_fits(p, (int)D, dtype), &id))) return rc;
-  if ((rc = device_check())) return rc;
+  if ((rc = check_config(TATTN_K_BWD_DKDV, D, dtype, config_id)) || (rc = device_check())) return rc;
+  const int id = config_id < 0 ? pick_bwd(TATTN_K_BWD_DKDV, p, (int)D, dtype, causal) : config_id;
   p.q = q; p.k = k; p.v = v; p.dout = dout; p.dk = dk; p.dv = dv; p.m = m; p.delta = const_cast<float*>(delta);
   return run_dkdv(p, (int)D, dtype, causal != 0, id, (hipStream_t)stream);
 }
@@ -452,9 +473,8 @@ static int bwd_dq_call(const void* q, const void* k, const void* v, const void* 
       (rc = check_tensor("dq", dq, strides, sz)))
     return rc;
   if (!m || !delta) return set_error(TATTN_E_ARG, "m and delta must not be null");
-  int id;
-  if ((rc = resolve(TATTN_K_BWD_DQ, D, dtype, causal, N, Z * H, config_id, bwd_own_fits(p, (int)D, dtype), &id))) return rc;
-  if ((rc = device_check())) return rc;
+  if ((rc = check_config(TATTN_K_BWD_DQ, D, dtype, config_id)) || (rc = device_check())) return rc;
+  const int id = config_id < 0 ? pick_bwd(TATTN_K_BWD_DQ, p, (int)D, dtype, causal) : config_id;
   p.q = q; p.k = k; p.v = v; p.dout = dout; p.dq = dq; p.m = m; p.delta = const_cast<float*>(delta);
   if (o_fused) {
     p.o = o_fused;
@@ -491,10 +511,8 @@ static int bwd_prepare(BwdParams& p, int* dk_id, int* dq_id, bool* fuse, const v
     if (config_id >= num_configs(TATTN_K_BWD_DKDV, D, dtype) || config_id >= num_configs(TATTN_K_BWD_DQ, D, dtype))
       return set_error(TATTN_E_CONFIG, "config id %d out of range for the backward tables", config_id);
   }
-  const bool own = bwd_own_fits(p, (int)D, dtype);
-  if ((rc = resolve(TATTN_K_BWD_DKDV, D, dtype, causal, N, Z * H, config_id, own, dk_id)) ||
-      (rc = resolve(TATTN_K_BWD_DQ, D, dtype, causal, N, Z * H, config_id, own, dq_id)))
-    return rc;
+  *dk_id = config_id < 0 ? pick_bwd(TATTN_K_BWD_DKDV, p, (int)D, dtype, causal) : config_id;
+  *dq_id = config_id < 0 ? pick_bwd(TATTN_K_BWD_DQ, p, (int)D, dtype, causal) : config_id;
   if ((rc = device_check())) return rc;
   // When dQ runs any kernel but the generic ones it computes delta itself
   // (same bits as the preprocess) and stores it: dQ, then dK/dV, two launches and no separate

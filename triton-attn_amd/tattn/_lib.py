@@ -23,8 +23,12 @@ KERNEL_NAMES = {K_FWD: "fwd", K_BWD_DKDV: "bwd_dkdv", K_BWD_DQ: "bwd_dq"}
 EXPORTS = (
     "tattn_abi_version", "tattn_last_error", "tattn_device_supported", "tattn_fwd",
     "tattn_bwd_preprocess", "tattn_bwd_dkdv", "tattn_bwd_dq", "tattn_bwd", "tattn_bwd_layouts", "tattn_bwd_noalloc",
-    "tattn_num_configs", "tattn_config_desc", "tattn_pick_config",
+    "tattn_num_configs", "tattn_config_desc", "tattn_pick_config", "tattn_picked",
 )
+
+# Kernels outside the tables, as `picked` reports them.
+PICK_COOP, PICK_PLANES, PICK_SHORT = 1000, 1001, 1002
+PICK_NAMES = {PICK_COOP: "coop", PICK_PLANES: "planes", PICK_SHORT: "short"}
 
 
 class TattnConfig(ctypes.Structure):
@@ -62,6 +66,7 @@ _SIGS = {
     "tattn_num_configs": (_I, [_I, _I64, _I]),
     "tattn_config_desc": (_I, [_I, _I64, _I, _I, ctypes.POINTER(TattnConfig)]),
     "tattn_pick_config": (_I, [_I, _I64, _I, _I, _I64]),
+    "tattn_picked": (_I, [_I, _STR4, _STR4, _I64, _I64, _I64, _I64, _I, _I, _F]),
 }
 
 _lib: ctypes.CDLL | None = None
@@ -143,4 +148,16 @@ def pick_config(kernel: int, d: int, dtype: int, causal: bool, n: int) -> int:
     rc = load().tattn_pick_config(kernel, d, dtype, int(causal), n)
     if rc < 0:
         raise RuntimeError(f"tattn_pick_config failed: {last_error()}")
+    return rc
+
+
+def picked(kernel: int, shape: tuple[int, int, int, int], dtype: int, causal: bool, *, scale: float | None = None,
+           strides: tuple[int, ...] | None = None, v_strides: tuple[int, ...] | None = None) -> int:
+    """What a call without a config runs: a table index or one of PICK_COOP, PICK_PLANES, PICK_SHORT.
+    `strides`: of k (forward; v's default to them) or shared by the backward's inputs; None: contiguous."""
+    z, h, n, d = shape
+    st, sv = ((ctypes.c_int64 * 4)(*x) if x is not None else None for x in (strides, v_strides))
+    rc = load().tattn_picked(kernel, st, sv, z, h, n, d, dtype, int(causal), d ** -0.5 if scale is None else scale)
+    if rc < 0:
+        raise RuntimeError(f"tattn_picked failed: {last_error()}")
     return rc

@@ -22,7 +22,8 @@ Result schema "tattn-suite/1":
     cells    [{impl, n, b, mask: "none"|"causal", pass: "fwd"|"fwd+bwd", status: "ok"|"oom"|
                "unsupported", ms, tflops, peak_mib, note}]
     errors   [{impl, n, mask, tensor: "o"|"dq"|"dk"|"dv", max_abs, mean_abs}]
-    gemm_tflops, picks {n/mask: {kernel: table id}}, autotuned (or null)
+    gemm_tflops, picks {n/mask: {kernel: table id, or the name of a kernel outside the tables}},
+    autotuned (or null)
 
 Render it with `python -m tattn.report FILE`.
 """
@@ -224,12 +225,17 @@ def gemm_rate() -> float:
     return 2 * 4096**3 / (do_bench(lambda: a @ b) * 1e-3) / 1e12
 
 
-def table_picks(seqs: Iterable[int], dim: int) -> dict[str, dict[str, int]]:
+def picks(seqs: Iterable[int], tokens: int, heads: int, dim: int) -> dict[str, dict[str, int | str]]:
+    """What each cell's call runs: a table index, or the name of a kernel outside the tables."""
     from . import _lib
 
-    return {f"{n}/{mask}": {name: _lib.pick_config(kid, dim, _lib.F16, mask == "causal", n)
-                            for kid, name in _lib.KERNEL_NAMES.items()}
-            for n in seqs for mask in MASKS}
+    out: dict[str, dict[str, int | str]] = {}
+    for n in seqs:
+        for mask in MASKS:
+            ids = {name: _lib.picked(kid, (max(1, tokens // n), heads, n, dim), _lib.F16, mask == "causal")
+                   for kid, name in _lib.KERNEL_NAMES.items()}
+            out[f"{n}/{mask}"] = {name: _lib.PICK_NAMES.get(cid, cid) for name, cid in ids.items()}
+    return out
 
 
 def run(seqs: list[int], tokens: int, heads: int, dim: int, autotune: bool = False,
@@ -253,7 +259,7 @@ def run(seqs: list[int], tokens: int, heads: int, dim: int, autotune: bool = Fal
         "cells": cells,
         "errors": errors,
         "gemm_tflops": gemm_rate(),
-        "picks": table_picks(seqs, dim),
+        "picks": picks(seqs, tokens, heads, dim),
         "autotuned": autotune_cache() if autotune else None,
     }
 
