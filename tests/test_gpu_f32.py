@@ -223,3 +223,29 @@ def test_tiny_rows_beside_ordinary_ones():
             assert ea <= 1.25 * eb + 2.0 ** -24 * r.norm().item(), (e, name)
         tiny = ref[1][:, :, ~ordinary]
         assert (got[1].double()[:, :, ~ordinary] - tiny).norm().item() <= rel * tiny.norm().item(), e
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("layout", ["one row", "rows 16 MiB apart", "tokens"])
+def test_both_directions_run_kernels_with_the_same_scores(layout, causal):
+    """Keys and values that the forward leaves to the block kernels while the backward's contiguous copies
+    would pass for the split ones, at scores of thousands, where M has to match the scores to their last bit:
+    attention's gradients are those of the block kernels given O and M."""
+    from tattn import _lib, attention
+    from tattn.api import _backward, _forward
+
+    n = 16 if layout == "rows 16 MiB apart" else 200
+    q, do = _rand((1, 4, n, 64), 1) * 30, _rand((1, 4, n, 64), 2)
+    if layout == "one row":
+        k, v = ((_rand((1, 4, 1, 64), 3 + s) * (30, 1)[s]).expand(1, 4, n, 64) for s in range(2))
+    elif layout == "tokens":
+        k, v = (_rand((1, n, 4, 64), 3 + s).transpose(1, 2) for s in range(2))
+    else:
+        k, v = (torch.empty_strided((1, 4, n, 64), (0, 64, 1 << 22, 1), device="cuda").copy_(_rand((1, 4, n, 64), 3 + s)) for s in range(2))
+    blocks = _lib.picked(_lib.K_FWD, (1, 4, n, 64), _lib.F32, causal, strides=k.stride(), v_strides=v.stride()) == 0
+    assert blocks == (layout != "tokens")
+    t = [x.detach().requires_grad_() for x in (q, k, v)]
+    got = torch.autograd.grad(attention(*t, causal=causal), t, do)
+    o, m = _forward(q, k, v, causal, 0.125)
+    want = _backward(q, k, v, o, m, do, causal, 0.125, config={"dkdv": 0, "dq": 0} if blocks else None)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))

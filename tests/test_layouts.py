@@ -80,7 +80,9 @@ def test_overlapping_rows(n, d, stride, dtype):
              for _ in range(5)]
     copies = [t.contiguous().clone() for t in views]
     _, m = _forward(copies[0], copies[1], copies[2], False, scale)
-    want = _backward(copies[0], copies[1], copies[2], copies[3], m, copies[4], False, scale)
+    # float32: the forward leaves such keys to the block kernels, and the backward follows it there.
+    blocks = {"dkdv": 0, "dq": 0} if dtype == torch.float32 else None
+    want = _backward(copies[0], copies[1], copies[2], copies[3], m, copies[4], False, scale, config=blocks)
     got = _backward(views[0], views[1], views[2], views[3], m, views[4], False, scale)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
     grads = [torch.empty_like(copies[0]) for _ in range(3)]

@@ -86,7 +86,9 @@ inline bool bwd_coop_fits(const BwdParams& p, int D, int dtype) {
 // causal, head dim 16: 5.4e-8 against 5.1e-8). So do short rows at
 // head dim 128, where one wave per SIMD is all that fits (us, forward / backward, split against block kernels:
 // 64 x 16 x 24: 41 / 159, 37 / 113; 64 x 8 x 64: 35 / 131, 37 / 119; 16 x 16 x 128 causal: 31 / 108, 40 / 122). Both
-// directions go the same way: M belongs to the bits of the forward's S.
+// directions have to go the same way, since M belongs to the bits of the forward's S: they do where K and V
+// of the forward and the inputs of the backward pass or fail alike, and a caller that copies in between (api.py) asks
+// for the block kernels by index where the forward ran them.
 int launch_fwd_f32(const FwdParams& p, int D, bool causal, hipStream_t st);
 int launch_dq_f32(const BwdParams& p, int D, bool causal, hipStream_t st);
 int launch_dkdv_f32(const BwdParams& p, int D, bool causal, hipStream_t st);

@@ -90,15 +90,18 @@ def _require_gpu(t: torch.Tensor) -> None:
 def _kernel_layout(t: torch.Tensor) -> torch.Tensor:
     """The kernels read rows with 16-byte vector loads: unit d stride, 16-byte aligned rows and
     base. Anything else is copied to a contiguous tensor (same values)."""
+    return t if _readable(t) else t.contiguous()
+
+
+def _readable(t: torch.Tensor) -> bool:
     if t.is_contiguous() and t.data_ptr() % 16 == 0:  # rows of 16+ elements: 16-byte multiples
-        return t
+        return True
     vec = 16 // t.element_size()
-    ok = (
+    return (
         t.stride(-1) == 1
         and all(s % vec == 0 for s in t.stride()[:3])
         and t.data_ptr() % 16 == 0
     )
-    return t if ok else t.contiguous()
 
 
 def _one_layout(q: torch.Tensor, *others: torch.Tensor) -> bool:
@@ -122,6 +125,19 @@ def _one_layout(q: torch.Tensor, *others: torch.Tensor) -> bool:
         and st[2] >= q.shape[3]
         and (q.shape[2] + 127) * st[2] * size < 1 << 31
     )
+
+
+def _forward_on_blocks(k: torch.Tensor, v: torch.Tensor, causal: bool, scale: float) -> bool:
+    """Whether the float32 forward left k and v as they lie (rows that overlap or lie far apart) to the
+    block kernels. The backward, which copies such inputs, has to stay with them: M goes with the
+    last bits of the forward's scores, and the kernels on split operands have others (one key 200 times, scores
+    near 3,900: dV off by 1.2e-5 of dO's norm instead of 1.5e-6)."""
+    if k.is_contiguous() and v.is_contiguous():
+        return False
+    z, h, n, d = k.shape
+    k_st, v_st = (t.stride() if _readable(t) else (h * n * d, n * d, d, 1) for t in (k, v))
+    return n > 0 and _lib.picked(_lib.K_FWD, (z, h, n, d), _lib.F32, causal, scale=scale, strides=k_st,
+                                 v_strides=v_st) != _lib.PICK_PLANES
 
 
 def _resolve(kernel: int, d: int, dtype: torch.dtype, config: Config, causal: bool, n: int) -> int:
@@ -263,6 +279,7 @@ def _backward(
     if do.dtype != q.dtype:
         do = do.to(q.dtype)
     whole = config is None and not _autotune  # one library call, which takes the inputs' own layout
+    pick = 0 if whole and q.dtype == torch.float32 and q.numel() and _forward_on_blocks(k, v, causal, scale) else -1
     if not (whole and _one_layout(q, k, v, do, o)):
         q, k, v, do, o = q.contiguous(), k.contiguous(), v.contiguous(), do.contiguous(), o.contiguous()
     m = m.contiguous()
@@ -272,12 +289,12 @@ def _backward(
         return dq, dk, dv
     code = _DTYPES[q.dtype]
     if whole:
-        # The whole backward in one library call: preprocess, dK/dV, dQ in stream order.
+        # The whole backward in one library call, in stream order.
         _, (st, gst) = _lib.stride_block(q, dq)
         with _on_device(q):
             rc = lib.tattn_bwd_layouts(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(),
                                        dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), m.data_ptr(), delta.data_ptr(),
-                                       st, gst, z, h, n, d, code, int(causal), float(scale), -1, _stream(q))
+                                       st, gst, z, h, n, d, code, int(causal), float(scale), pick, _stream(q))
         _lib.check(rc, "tattn_bwd")
         return dq, dk, dv
     _, (st,) = _lib.stride_block(q)
