@@ -178,3 +178,12 @@ def test_picked_names_the_kernel_that_a_call_runs(kernel):
         pick((1, 1, 16, 48), _lib.F16)
     with pytest.raises(RuntimeError, match="no kernel"):
         _lib.picked(7, (1, 1, 16, 64), _lib.F16, False)
+
+
+def test_picks_stay_within_what_a_launch_may_have():
+    """The kernels that split the summed dimension take eight threads per row; a launch takes fewer than 2^32."""
+    assert _lib.picked(_lib.K_BWD_DQ, (1 << 10, 16, 1024, 32), _lib.F16, True) == _lib.PICK_COOP
+    for kernel in (_lib.K_FWD, _lib.K_BWD_DKDV, _lib.K_BWD_DQ):
+        for d in (16, 32, 64, 128):
+            for causal in (False, True):
+                assert _lib.picked(kernel, (1 << 15, 16, 1024, d), _lib.F16, causal) < _lib.num_configs(kernel, d, _lib.F16)

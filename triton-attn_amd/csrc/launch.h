@@ -68,16 +68,19 @@ inline bool bwd_short_fits(const BwdParams& p, int D, int dtype) {
 }
 
 // Waves of a workgroup split the summed dimension (coop.hip); 16-bit, slices that fit 32-bit
-// offsets, and for the forward a scale other than 0 (it hides keys at a score whose scaled value is -inf).
+// offsets, fewer than the 2^32 threads that a launch may have (eight per row, where the block kernels take two),
+// and for the forward a scale other than 0 (it hides keys at a score whose scaled value is -inf).
 int launch_fwd_coop(const FwdParams& p, int D, int dtype, bool causal, hipStream_t st);
 int launch_dq_coop(const BwdParams& p, int D, int dtype, bool causal, hipStream_t st);
 int launch_dkdv_coop(const BwdParams& p, int D, int dtype, bool causal, hipStream_t st);
+inline bool coop_launches(int64_t Z, int64_t H, int64_t N) { return Z * H * ((N + 63) / 64) * 512 < (1ll << 32); }
 inline bool fwd_coop_fits(const FwdParams& p, int D, int dtype) {
-  return dtype != 1 && p.c != 0.0f && slice_bytes(p.N, p.sk[2], D) + (uint64_t)p.sk[2] * 128 < (1ull << 31) &&
+  return dtype != 1 && p.c != 0.0f && coop_launches(p.Z, p.H, p.N) &&
+         slice_bytes(p.N, p.sk[2], D) + (uint64_t)p.sk[2] * 128 < (1ull << 31) &&
          slice_bytes(p.N, p.sv[2], D) + (uint64_t)p.sv[2] * 128 < (1ull << 31) && (p.sk[2] | p.sv[2]) < (1ll << 22);
 }
 inline bool bwd_coop_fits(const BwdParams& p, int D, int dtype) {
-  return dtype != 1 && bwd_fits32(p, D) && p.s[2] < (1ll << 22);
+  return dtype != 1 && coop_launches(p.Z, p.H, p.N) && bwd_fits32(p, D) && p.s[2] < (1ll << 22);
 }
 
 // float32 on split operands (f32_split.hip): row offsets of a slice, with a step's look-ahead, fit 32
