@@ -187,3 +187,12 @@ def test_picks_stay_within_what_a_launch_may_have():
         for d in (16, 32, 64, 128):
             for causal in (False, True):
                 assert _lib.picked(kernel, (1 << 15, 16, 1024, d), _lib.F16, causal) < _lib.num_configs(kernel, d, _lib.F16)
+
+
+@pytest.mark.parametrize("kernel", [_lib.K_FWD, _lib.K_BWD_DQ])
+@pytest.mark.parametrize("causal", [False, True])
+def test_slices_read_by_every_xcd_stay_with_the_block_kernels(kernel, causal):
+    """Z*H not a multiple of 8 and more K and V than the caches hold."""
+    for zh in (37, 113):
+        assert _lib.picked(kernel, (1, zh, 4505, 128), _lib.F16, causal) < _lib.num_configs(kernel, 128, _lib.F16)
+    assert _lib.picked(kernel, (1, 3, 2049, 128), _lib.F16, causal) == _lib.PICK_COOP

@@ -100,20 +100,31 @@ const TileEntry* config_entry(int kernel, int64_t D, int dtype, int id) {
 }
 
 // What a launch costs in rows of one CU: workgroups of `rows` rows are dealt to the 256 CUs, and the
-// CU with the most of them sets the time. `eff`: measured time per row against the fastest kernel
-// when the chip is full; `alone`: what a single workgroup of four waves on a CU (one wave per SIMD)
-// loses on top. Without a mask all workgroups of a launch are equal and this ranks the kernels
-// within a few percent (fp16, 1,000 to 8,192 row tiles, N = 500 to 12,345: e.g. forward, head dim 64,
-// 12 slices x 12,345 rows: 512-row blocks 1,024 CU rows 700 us, 256-row 768 569 us, 128-row 640
-// 530 us; 16 x 2,048: 512 59 us, 256 38 us, 128 26 us).
+// CU with the most of them sets the time. `eff`: measured time per row where CUs hold several workgroups;
+// `alone`: what a single workgroup on a CU loses (or gains, above 128 rows) on top. Without a mask all
+// workgroups of a launch are equal, and this ranks the kernels: the constants below were fitted to the times of
+// every entry at 871 shapes at head dim 64, 769 at 128, 451 at 32 and 417 at 16 (fp16, N = 129 to 12,000, up to 300,000
+// rows). There the pick is on average 0.5 to 2% behind the fastest entry. Of 3,592 launches at other shapes 1.2% were
+// more than 3% slower than the picks by length alone that these replace, two more than 10%; on average those took 1.26
+// times as long. (Causal, with the tile counts below: 4,797 launches, 0.2%, none, 1.38.)
 double cu_rows(int64_t ZH, int64_t N, int rows, double eff, double alone = 1.0) {
   const int64_t k = (ZH * ((N + rows - 1) / rows) + 255) / 256;
   return (double)(k * rows) * eff * (k == 1 ? alone : 1.0);
 }
 
-// The same for coop.hip's kernels, whose prologue and final merge weigh on short rows (9 x 16 x 396:
-// 10-20% behind the block kernels where the row count alone puts them ahead).
-double coop_rows(int64_t ZH, int64_t N, double eff) { return cu_rows(ZH, N, 64, eff * (1.0 + 128.0 / (double)N)); }
+// The same for coop.hip's kernels (64 rows), whose prologue and final merge weigh on short rows as `head`
+// more rows would.
+double coop_rows(int64_t ZH, int64_t N, double eff, double head, double alone = 1.0) {
+  return cu_rows(ZH, N, 64, eff * (1.0 + head / (double)N), alone);
+}
+
+// Those kernels read K and V (Q and dO) once per 64 rows, the others once per 128 or 256. Where ZH is not a
+// multiple of 8 a slice is read by every XCD, and once the slices outgrow the L2s that costs them half their time or
+// more (head dim 128, us, coop against paired waves / pipelined: dQ 37 x 4,505 822 / 664, causal 113 x 1,556 189 / 154;
+// forward 21 x 2,038 79 / 66; head dim 64 causal forward, 53 x 1,235: 31.7 / 26.0): not picked there above this many bytes of K and V.
+bool coop_in_reach(int64_t ZH, int64_t N, int64_t D, bool causal) {
+  return ZH % 8 == 0 || ZH * N * D * 4 <= ((causal ? 12 : 24) << 20);
+}
 
 // The cheapest of a few candidates; the first wins ties.
 struct Cheapest {
@@ -135,17 +146,17 @@ constexpr int kCoop = TATTN_PICK_COOP, kSplit = TATTN_PICK_PLANES, kShort = TATT
 // general-purpose tile. Persistent entries are picked where they run the problem themselves.
 //
 // Causal launches are bound by their longest workgroups when the chip is not full: coop (a quarter
-// of the chain) up to a number of 32-row tiles, measured per kernel and head dim (us, coop against
-// the best other entry, N = 1,177 to 12,345):
-//   forward   64: 2,256 tiles 27.7 / 28.3, 6,000 134 / 126   128: 1,776 32.9 / 33.4, 2,256 46 / 42
-//             32: 6,000 82 / 83, 6,204 46 / 43
-//   dQ        64: 1,024 23 / 30, 1,760 95 / 118, 1,776 (N = 1,177) 31 / 26   128: 6,000 299 / 323, 6,204 170 / 167
-//             32: every size (8,192 tiles 51 / 53) from N = 768
-//   dK/dV     64: 1,024 31 / 45, 1,760 128 / 149, 1,776 (N = 1,177) 45 / 31   32: 4,632 299 / 314, 6,204 71 / 66, N = 384: 3,648 22 / 15
-//             128: never (its registers spill there)
+// of the chain) up to a number of 32-row tiles, fewer on short rows, where the chain is short as well.
+// Measured per kernel and head dim (us, coop against the entry picked otherwise, N = 129 to 12,345):
+//   forward   64: 2,256 tiles 27.7 / 28.3, 6,000 134 / 126, 1,784 (N = 256) 15.3 / 13.0, 2,128 (512) 23.8 / 19.9
+//             128: 1,776 32.9 / 33.4, 2,256 46 / 42   32: 6,000 82 / 83, 6,204 46 / 43
+//   dQ        64: 1,024 23 / 30, 1,760 95 / 118, 1,776 (1,177) 31 / 26   128: 6,000 299 / 323, 6,204 170 / 167
+//             32: every size (8,192 tiles 51 / 53) from N = 768   16: 5,632 (1,024) 28.1 / 25.9, 3,072 (768) 14.4 / 12.6
+//   dK/dV     64: 1,024 31 / 45, 1,760 128 / 149, 1,776 (1,177) 45 / 31   32: 4,632 299 / 314, 6,204 71 / 66, N = 384: 3,648 22 / 15
+//             16: 3,408 (2,242) 45.8 / 41.2, 4,128 (4,104) 87.7 / 77.6   128: never (its registers spill there)
 int pick_config(int kernel, int64_t D, int dtype, int causal, int64_t N, int64_t ZH, bool own) {
   if (dtype == TATTN_F32) return own ? kSplit : 0;  // fp16 and bf16 share the picks
-  bool coop = own;
+  bool coop = own && coop_in_reach(ZH, N, D, causal != 0);
   const int64_t tiles = ZH * ((N + 31) / 32);
   Cheapest best;
   switch (kernel) {
@@ -156,7 +167,7 @@ int pick_config(int kernel, int64_t D, int dtype, int causal, int64_t N, int64_t
       // than the flat flip allowance that the stress tests (2 x 1,024 rows) state. It would take
       // 9 us where 1 x 1,024 x 64 takes 21.
       coop = coop && tiles >= 96;
-      const int64_t coop_most = D == 64 ? 2304 : D == 128 ? 1800 : 6144;
+      const int64_t coop_most = D == 64 ? std::min<int64_t>(2304, N * 2) : D == 128 ? 1800 : 6144;
       if (causal && coop && tiles <= coop_most) return kCoop;
       if (causal) {
         if (D == 64) {
@@ -175,28 +186,33 @@ int pick_config(int kernel, int64_t D, int dtype, int causal, int64_t N, int64_t
       }
       if (D == 64) {
         // Persistent 4 x 2 and 4 x 1 (ring of 4), pipelined 4 x 2, 8 x 2 from N = 4096, 4 x 1.
-        if (fwd_persist_fits(FwdTable<_Float16, 64>::e[7], ZH, N, false)) best.offer(7, cu_rows(ZH, N, 256, 0.95));
-        if (fwd_persist_fits(FwdTable<_Float16, 64>::e[5], ZH, N, false)) best.offer(5, cu_rows(ZH, N, 128, 1.07, 1.4));
-        best.offer(0, cu_rows(ZH, N, 256, 1.0));
+        if (fwd_persist_fits(FwdTable<_Float16, 64>::e[7], ZH, N, false)) best.offer(7, cu_rows(ZH, N, 256, 0.86, 1.21));
+        if (fwd_persist_fits(FwdTable<_Float16, 64>::e[5], ZH, N, false)) best.offer(5, cu_rows(ZH, N, 128, 0.99, 1.47));
+        best.offer(0, cu_rows(ZH, N, 256, 1.0, 1.13));
         if (N >= 4096) best.offer(3, cu_rows(ZH, N, 512, 0.99));
-        best.offer(1, cu_rows(ZH, N, 128, 1.06, 1.4));
-        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.4));
+        best.offer(1, cu_rows(ZH, N, 128, 1.02, 1.39));
+        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.29, 128, 1.2));
       } else if (D == 128) {
         // Persistent 8 x 1 from N = 2048, 4 x 1; pipelined 4 x 1.
         if (N >= 2048 && fwd_persist_fits(FwdTable<_Float16, 128>::e[3], ZH, N, false))
-          best.offer(3, cu_rows(ZH, N, 256, 0.96));
+          best.offer(3, cu_rows(ZH, N, 256, 0.72));
         if (fwd_persist_fits(FwdTable<_Float16, 128>::e[2], ZH, N, false)) best.offer(2, cu_rows(ZH, N, 128, 1.0, 1.1));
-        best.offer(0, cu_rows(ZH, N, 128, 1.02));
-        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.25));
+        best.offer(0, cu_rows(ZH, N, 128, 1.04, 1.05));
+        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.4, 64));
+      } else if (D == 32) {
+        best.offer(0, cu_rows(ZH, N, 256, 0.98, 1.06));
+        best.offer(1, cu_rows(ZH, N, 128, 1.01, 1.41));
+        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.1, 96));
       } else {
-        best.offer(0, cu_rows(ZH, N, 256, 1.0));
-        best.offer(1, cu_rows(ZH, N, 128, D == 16 && N < 2048 ? 0.99 : 1.06, 1.4));
-        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.2));
+        best.offer(0, cu_rows(ZH, N, 256, 1.06, 1.19));
+        best.offer(1, cu_rows(ZH, N, 128, 1.14, 1.37));
+        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.11, 128));
       }
       return best.id;
     }
     case TATTN_K_BWD_DKDV: {
-      const int64_t coop_most = D == 64 ? std::min<int64_t>(1800, N * 3 / 4) : D == 128 ? 0 : std::min<int64_t>(4800, N * 8 / 5);
+      const int64_t coop_most = D == 64 ? std::min<int64_t>(1800, N * 3 / 4) : D == 128 ? 0
+                              : std::min<int64_t>(D == 16 ? 3000 : 4800, N * 8 / 5);
       if (causal && coop && tiles <= coop_most) return kCoop;
       // Paired waves at head dim 128: two per SIMD, where one wave per tile needs all 512 registers.
       if (D == 128) return 2;
@@ -209,33 +225,44 @@ int pick_config(int kernel, int64_t D, int dtype, int causal, int64_t N, int64_t
         return N >= 2048 ? 1 : 0;
       }
       if (D == 64) {
-        best.offer(1, cu_rows(ZH, N, 256, 1.0));
-        best.offer(0, cu_rows(ZH, N, 128, 1.35, 1.2));  // streams Q and dO past twice as many blocks
-        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.4 + 180.0 / (double)N));
+        best.offer(1, cu_rows(ZH, N, 256, 0.93, 0.91));
+        best.offer(0, cu_rows(ZH, N, 128, 1.38, 1.2));  // streams Q and dO past twice as many blocks
+        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.4, 180, 1.21));
+      } else if (D == 32) {
+        best.offer(0, cu_rows(ZH, N, 128, 1.11, 1.58));
+        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.15, 180));
       } else {
-        best.offer(0, cu_rows(ZH, N, 128, 1.0, 1.4));
-        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.15));
+        best.offer(0, cu_rows(ZH, N, 128, 1.05, 1.83));
+        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.1, 128));
       }
       return best.id;
     }
     case TATTN_K_BWD_DQ: {
-      // Head dims 16, 32: coop, except many short rows (16 x 16 x 384 causal: 13.6 against 12.7 us).
-      if (D < 64) return coop && (N >= (causal || D == 16 ? 768 : 448) || tiles <= N * 8 / 5) ? kCoop : 0;
-      const int64_t coop_most = D == 64 ? std::min<int64_t>(1800, N * 6 / 5) : 6000;
+      if (causal && D < 64) {
+        // Coop, except many short rows (32: 16 x 16 x 384 13.6 against 12.7 us) and, at 16, full chips.
+        if (D == 16) return coop && tiles <= std::min<int64_t>(5000, N * 3) ? kCoop : 0;
+        return coop && (N >= 768 || tiles <= N * 8 / 5) ? kCoop : 0;
+      }
+      const int64_t coop_most = D == 64 ? std::min<int64_t>(1700, N * 6 / 5) : std::min<int64_t>(6000, N * 8);
       if (causal && coop && tiles <= coop_most) return kCoop;
       if (D == 128) {  // paired waves, as dK/dV
         if (causal) return 2;
-        best.offer(2, cu_rows(ZH, N, 128, 1.0));
-        if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.05));
+        best.offer(2, cu_rows(ZH, N, 128, 1.07, 0.96));
+        if (coop) best.offer(kCoop, coop_rows(ZH, N, 0.95, 64));
+        return best.id;
+      }
+      if (D < 64) {
+        best.offer(0, D == 32 ? cu_rows(ZH, N, 128, 1.03, 1.33) : cu_rows(ZH, N, 128, 1.02, 2.08));
+        if (coop) best.offer(kCoop, D == 32 ? coop_rows(ZH, N, 0.82, 128) : coop_rows(ZH, N, 0.93, 180));
         return best.id;
       }
       // Persistent 4 waves where it fits; pipelined 4 or 8 waves.
       const bool persist = bwd_persist_fits(DqTable<_Float16, 64>::e[5], ZH, N, causal != 0);
       if (causal) return persist ? 5 : 0;
-      if (persist) best.offer(5, cu_rows(ZH, N, 128, 0.95, 1.2));
-      best.offer(0, cu_rows(ZH, N, 128, 1.02, 1.2));
-      best.offer(1, cu_rows(ZH, N, 256, 1.06));
-      if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.25));
+      if (persist) best.offer(5, cu_rows(ZH, N, 128, 0.92, 1.2));
+      best.offer(0, cu_rows(ZH, N, 128, 1.02, 1.35));
+      best.offer(1, cu_rows(ZH, N, 256, 1.06, 0.87));
+      if (coop) best.offer(kCoop, coop_rows(ZH, N, 1.16, 180, 0.92));
       return best.id;
     }
   }
