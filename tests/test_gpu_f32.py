@@ -60,6 +60,18 @@ def test_split_kernels_against_float64(z, h, n, d, causal):
 
 
 @pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [16, 32, 64, 128])
+@pytest.mark.parametrize("z,h,n", [(65, 8, 4), (65, 8, 24), (33, 8, 33), (2, 3, 41), (100, 1, 146), (47, 1, 400), (16, 1, 1100)])
+def test_split_kernels_at_the_edges_of_their_picks(z, h, n, d, causal):
+    """Two slices per CU and short rows; around one workgroup per CU at head dim 128."""
+    from tattn import _lib
+
+    for kernel in (_lib.K_FWD, _lib.K_BWD_DKDV, _lib.K_BWD_DQ):
+        assert (_lib.picked(kernel, (z, h, n, d), _lib.F32, causal) == _lib.PICK_PLANES) == (d < 128 or n > 96)
+    _compare(*(_rand((z, h, n, d), n + s) for s in range(4)), causal, d ** -0.5)
+
+
+@pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("scale", [-0.125, 0.0, 0.5])
 def test_scales(scale, causal):
     _compare(*(_rand((2, 8, 300, 64), 50 + s) for s in range(4)), causal, scale)
@@ -85,7 +97,17 @@ def test_magnitudes(mag):
 @pytest.mark.parametrize("n", [40, 200, 600])
 @pytest.mark.parametrize("causal", [False, True])
 def test_infinities_and_nans_go_where_the_block_kernels_take_them(causal, n):
-    q, k, v, do = (_rand((2, 8, n, 64), 30 + s) for s in range(4))
+    _infinities_and_nans(2, n, causal)
+
+
+@pytest.mark.parametrize("n", [31, 60])
+@pytest.mark.parametrize("causal", [False, True])
+def test_infinities_and_nans_in_short_rows(causal, n):
+    _infinities_and_nans(65, n, causal)
+
+
+def _infinities_and_nans(z, n, causal):
+    q, k, v, do = (_rand((z, 8, n, 64), 30 + s) for s in range(4))
     q[0, 1, 17, 5] = float("nan")
     k[0, 2, 3, 7] = float("-inf")  # hides key 3 from queries whose component is positive
     v[0, 3, 9, 11] = float("inf")
@@ -138,7 +160,7 @@ def _hidden_keys(shape, causal, scale, hide, low, q0):
 
 
 # Waves per row tile and tiles per step: {2, 4}, {4, 2}, {4, 1}, {1, 1}; head dim 128 {2, 2}, {4, 1}.
-SHAPES = [(2, 4, 128, 64), (4, 16, 512, 64), (40, 16, 512, 64), (2, 3, 30, 32), (1, 8, 600, 128), (16, 16, 600, 128)]
+SHAPES = [(2, 4, 128, 64), (4, 16, 512, 64), (40, 16, 512, 64), (65, 8, 30, 32), (1, 8, 600, 128), (16, 16, 600, 128)]
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))

@@ -854,7 +854,14 @@ Pick pick_shape(int D, int64_t zh, int64_t n, bool causal, bool backward) {
     const int64_t k = ((int64_t)wgs + 255) / 256;
     return steps * ((double)(k / 2) * two + (double)(k % 2) * one) + merge;
   };
-  if (D == 128) return cost(2, 2, 5.9, 11.8, 5.9, 1.6) < cost(4, 1, 4.0, 8.0, 4.0, 0.0) ? FEW : ROWS;
+  if (D == 128) {
+    // Causal, {2, 2}: one workgroup fills a CU, and with more workgroups than CUs some CU gets two long ones unless
+    // the chain is long (against {4, 1}, us, forward / backward: 100 x 146 35 / 166, 27 / 117; 3,000 x 146 706 / 3,533,
+    // 597 / 2,455; 64 x 400 58 / 263, 57 / 240; 32 x 800 82 / 350, 102 / 411; 16 x 2,048 203 / 854, 256 / 1,006).
+    const int64_t wgs = zh * ((n + 63) / 64);
+    if (causal && wgs > 256 && (n <= 256 || wgs > (backward && n < 768 ? 384 : 512))) return ROWS;
+    return cost(2, 2, 5.9, 11.8, 5.9, 1.6) < cost(4, 1, 4.0, 8.0, 4.0, 0.0) ? FEW : ROWS;
+  }
   const double rows = cost(4, 1, 2.0, 3.2, 2.0, 0.0), half = cost(4, 2, 3.2, 6.4, 2.8, 1.6), few = cost(2, 4, 4.2, 8.4, 3.6, 1.6);
   return few < rows && few < half ? FEW : half < rows ? HALF : ROWS;
 }

@@ -86,20 +86,29 @@ inline bool bwd_coop_fits(const BwdParams& p, int D, int dtype) {
 // float32 on split operands (f32_split.hip): row offsets of a slice, with a step's look-ahead, fit 32
 // bits, and rows past the end of a slice lie past its last element (rows that overlap do not). One to three
 // keys stay with the block kernels: sums of so few products are no closer to float64 here (dV of 2 keys,
-// causal, head dim 16: 5.4e-8 against 5.1e-8). So do short rows at
-// head dim 128, where one wave per SIMD is all that fits (us, forward / backward, split against block kernels:
-// 64 x 16 x 24: 41 / 159, 37 / 113; 64 x 8 x 64: 35 / 131, 37 / 119; 16 x 16 x 128 causal: 31 / 108, 40 / 122). Both
+// causal, head dim 16: 5.4e-8 against 5.1e-8). So do, where they are the faster ones (us, forward / backward, split
+// against block kernels):
+//   head dim 128 up to 96 rows, where one wave per SIMD is all that fits (64 x 16 x 24: 41 / 159, 37 / 113; 64 x 8 x 64:
+//   35 / 131, 37 / 119; 16 x 16 x 128 causal: 31 / 108, 40 / 122);
+//   32 and 64 up to 32 rows with at most two slices per CU and up to 40 with one, where one wave stages and splits
+//   what four share there (64: 47 x 26 8.5 / 22.3, 6.0 / 19.2; 520 x 32 10.0 / 25.7, 11.4 / 39.1; 256 x 40 9.3 / 33.8,
+//   9.8 / 30.8; 260 x 40 10.6 / 33.8, 14.3 / 47.8; 32: 256 x 16 5.9 / 14.2, 4.8 / 12.7).
+// Both
 // directions have to go the same way, since M belongs to the bits of the forward's S: they do where K and V
 // of the forward and the inputs of the backward pass or fail alike, and a caller that copies in between (api.py) asks
 // for the block kernels by index where the forward ran them.
 int launch_fwd_f32(const FwdParams& p, int D, bool causal, hipStream_t st);
 int launch_dq_f32(const BwdParams& p, int D, bool causal, hipStream_t st);
 int launch_dkdv_f32(const BwdParams& p, int D, bool causal, hipStream_t st);
-inline bool f32_rows_fit(int64_t N, int64_t row_stride, int D) {
-  return N > (D < 128 ? 3 : 96) && row_stride >= D && row_stride < (1ll << 22) && (N + 256) * row_stride * 4 < (1ll << 31);
+inline bool f32_rows_fit(int64_t ZH, int64_t N, int64_t row_stride, int D) {
+  const int64_t most = D == 128 ? 96 : D < 32 || ZH > 512 ? 3 : ZH > 256 ? 32 : 40;  // rows of the block kernels
+  return N > most && row_stride >= D && row_stride < (1ll << 22) && (N + 256) * row_stride * 4 < (1ll << 31);
 }
-inline bool fwd_f32_fits(const FwdParams& p, int D) { return f32_rows_fit(p.N, p.sk[2], D) && f32_rows_fit(p.N, p.sv[2], D); }
-inline bool bwd_f32_fits(const BwdParams& p, int D) { return f32_rows_fit(p.N, p.s[2], D); }
+inline bool fwd_f32_fits(const FwdParams& p, int D) {
+  const int64_t zh = (int64_t)p.Z * p.H;
+  return f32_rows_fit(zh, p.N, p.sk[2], D) && f32_rows_fit(zh, p.N, p.sv[2], D);
+}
+inline bool bwd_f32_fits(const BwdParams& p, int D) { return f32_rows_fit((int64_t)p.Z * p.H, p.N, p.s[2], D); }
 
 // Compute units of the current device (cached per device).
 inline int device_cus() {
