@@ -87,6 +87,37 @@ def test_autotune_first_use_times_once_and_stays_correct(monkeypatch):
             assert 0 <= cid < real(kid, 64, _lib.F16)
 
 
+def test_autotune_keeps_kernels_outside_the_table(monkeypatch):
+    """Timing takes the library's pick as a candidate: for many short rows, where it is several times as fast
+    as every table entry, both directions keep it (the backward as one call, inputs in place), and float32,
+    which is not timed, gives the default's bits."""
+    import tattn
+    from tattn import _lib, api
+
+    for name in ("_tuned", "_pick_wins", "_whole_wins"):
+        monkeypatch.setattr(api, name, {})
+
+    def run(shape, dtype):
+        q, k, v, do = (rand(shape, dtype, 40 + s, DEV).transpose(1, 2) for s in range(4))
+        t = [x.detach().requires_grad_() for x in (q, k, v)]
+        o = tattn.attention(*t)
+        return (o.detach(), *torch.autograd.grad(o, t, do))
+
+    short, full = ((256, 24, 64, 16), torch.float16), ((2, 300, 8, 64), torch.float32)
+    want = run(*short), run(*full)
+    tattn.set_autotune(True)
+    try:
+        for _ in range(2):  # timed, then kept
+            got = run(*short), run(*full)
+            for a, b in zip((*got[0], *got[1]), (*want[0], *want[1])):
+                assert torch.equal(a, b)
+    finally:
+        tattn.set_autotune(False)
+    assert list(api._whole_wins.values()) == [True]
+    assert [won for key, won in api._pick_wins.items() if key[0] == _lib.K_FWD] == [True]
+    assert all(key[4] == _lib.F16 for key in api._tuned)
+
+
 def _raw_backward(kernel, q, k, v, do, m, delta, causal, cid):
     """One dK/dV or dQ launch through the C ABI with a given table entry."""
     from tattn import _lib

@@ -186,14 +186,18 @@ def _on_device(t: torch.Tensor):
     return contextlib.nullcontext() if idx == _current_device() else torch.cuda.device(idx)
 
 
-# Optional first-use timing of the tile table. The reference autotunes on the first call of each
+# Optional first-use timing. The reference autotunes on the first call of each
 # (N bucket, head dim, causal) key (src/tattn/kernels.py:57-61, 151-155, 242-246); here the
 # measured picks of the library are the default and timing is opt-in: TATTN_AUTOTUNE=1 in the
-# environment, or set_autotune(True). The first call of a key then times every table entry on
-# the caller's stream (HIP events; skipped while a graph is being captured) and keeps the
-# fastest for that key.
+# environment, or set_autotune(True). The first call of a key then times every table entry and the
+# library's own pick, which may be a kernel outside the table, on the caller's stream (HIP events; skipped
+# while a graph is being captured) and keeps the fastest for that key; the backward also times the pick's
+# single library call against its own three launches. float32 keeps to the library's picks, which send
+# both directions to kernels with the same scores.
 _autotune = os.environ.get("TATTN_AUTOTUNE", "0") not in ("", "0")
 _tuned: dict[tuple[int, int, int, int, int, bool], int] = {}  # (kernel, device, N bucket, D, dtype, causal)
+_pick_wins: dict[tuple[int, int, int, int, int, bool], bool] = {}  # the same keys: the library's pick is faster
+_whole_wins: dict[tuple[int, int, int, int, bool], bool] = {}  # (device, ...): so is the backward in one call
 
 
 def set_autotune(on: bool) -> None:
@@ -203,8 +207,9 @@ def set_autotune(on: bool) -> None:
 
 
 def autotune_cache() -> dict[str, dict[str, int]]:
-    """Entries chosen by timing so far: {kernel: {"device=.., n_bucket=.., d=.., dtype=..,
-    causal=..": table id}} (the analog of the reference bench's dump of its autotune caches)."""
+    """The fastest table entry by timing so far: {kernel: {"device=.., n_bucket=.., d=.., dtype=..,
+    causal=..": table id}} (the analog of the reference bench's dump of its autotune caches). Calls use
+    the library's own pick instead where that was faster still."""
     out: dict[str, dict[str, int]] = {name: {} for name in _lib.KERNEL_NAMES.values()}
     for (kernel, dev, bucket, d, code, causal), cid in _tuned.items():
         dtype = str({c: t for t, c in _DTYPES.items()}[code]).removeprefix("torch.")
@@ -213,31 +218,34 @@ def autotune_cache() -> dict[str, dict[str, int]]:
     return out
 
 
+def _launches_ms(launch: Callable[[], int], stream: torch.cuda.Stream) -> float:
+    """Time of three launches after one untimed; infinity where the call refuses."""
+    if launch() != 0:
+        return float("inf")
+    start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    start.record(stream)
+    for _ in range(3):
+        launch()
+    end.record(stream)
+    end.synchronize()
+    return start.elapsed_time(end)
+
+
 def _tuned_id(kernel: int, t: torch.Tensor, d: int, causal: bool, n: int,
               launch: Callable[[int], int]) -> int:
-    """The table entry for this call: -1 (the library's pick) unless autotuning is on; then the
-    fastest entry for the key, timed on first use by running `launch(id)` for every entry."""
-    if not _autotune or torch.cuda.is_current_stream_capturing():
+    """What this call runs: -1 (the library's pick) unless autotuning is on; then the fastest of the
+    table's entries and the pick for the key, timed on first use by running `launch(id)` for each."""
+    if not _autotune or t.dtype == torch.float32 or torch.cuda.is_current_stream_capturing():
         return -1
     code = _DTYPES[t.dtype]
     key = (kernel, t.device.index or 0, _bucket(n), d, code, causal)
     if key not in _tuned:
         stream = torch.cuda.current_stream(t.device)
-        best, best_ms = -1, float("inf")
-        for cid in range(_lib.num_configs(kernel, d, code)):
-            if launch(cid) != 0:  # not usable for this call: skip
-                continue
-            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            start.record(stream)
-            for _ in range(3):
-                launch(cid)
-            end.record(stream)
-            end.synchronize()
-            ms = start.elapsed_time(end)
-            if ms < best_ms:
-                best, best_ms = cid, ms
+        ms = {cid: _launches_ms(lambda: launch(cid), stream) for cid in range(_lib.num_configs(kernel, d, code))}
+        best = min(ms, key=ms.__getitem__)
+        _pick_wins[key] = _launches_ms(lambda: launch(-1), stream) <= ms[best]
         _tuned[key] = best
-    return _tuned[key]
+    return -1 if _pick_wins.get(key, False) else _tuned[key]
 
 
 def _forward(
@@ -278,7 +286,13 @@ def _backward(
     z, h, n, d = q.shape
     if do.dtype != q.dtype:
         do = do.to(q.dtype)
-    whole = config is None and not _autotune  # one library call, which takes the inputs' own layout
+    code = _DTYPES[q.dtype]
+    tuning = (
+        config is None and _autotune and q.dtype != torch.float32 and not torch.cuda.is_current_stream_capturing()
+    )
+    tune_key = (q.device.index or 0, _bucket(n), d, code, causal) if tuning else None
+    # One library call, which takes the inputs' own layout.
+    whole = config is None and (tune_key is None or _whole_wins.get(tune_key, False))
     pick = 0 if whole and q.dtype == torch.float32 and q.numel() and _forward_on_blocks(k, v, causal, scale) else -1
     if not (whole and _one_layout(q, k, v, do, o)):
         q, k, v, do, o = q.contiguous(), k.contiguous(), v.contiguous(), do.contiguous(), o.contiguous()
@@ -287,7 +301,6 @@ def _backward(
     dq, dk, dv = q.new_empty(q.shape), q.new_empty(q.shape), q.new_empty(q.shape)
     if q.numel() == 0:
         return dq, dk, dv
-    code = _DTYPES[q.dtype]
     if whole:
         # The whole backward in one library call, in stream order.
         _, (st, gst) = _lib.stride_block(q, dq)
@@ -308,13 +321,28 @@ def _backward(
                  m.data_ptr(), delta.data_ptr(), st, z, h, n, d, code, int(causal), float(scale))
     dq_args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), do.data_ptr(), dq.data_ptr(), m.data_ptr(),
                delta.data_ptr(), st, z, h, n, d, code, int(causal), float(scale))
+    pre_args = (o.data_ptr(), do.data_ptr(), delta.data_ptr(), st, z, h, n, d, code)
     with _on_device(q):
         stream = _stream(q)
-        _lib.check(lib.tattn_bwd_preprocess(o.data_ptr(), do.data_ptr(), delta.data_ptr(), st,
-                                            z, h, n, d, code, stream), "tattn_bwd_preprocess")
-        if config is None:
+        _lib.check(lib.tattn_bwd_preprocess(*pre_args, stream), "tattn_bwd_preprocess")
+        if tune_key is not None:
             kid = _tuned_id(_lib.K_BWD_DKDV, q, d, causal, n, lambda c: lib.tattn_bwd_dkdv(*dkdv_args, c, stream))
             qid = _tuned_id(_lib.K_BWD_DQ, q, d, causal, n, lambda c: lib.tattn_bwd_dq(*dq_args, c, stream))
+            if tune_key not in _whole_wins:
+                def one() -> int:
+                    return lib.tattn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(),
+                                         dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), m.data_ptr(), delta.data_ptr(),
+                                         st, z, h, n, d, code, int(causal), float(scale), -1, stream)
+
+                def three() -> int:
+                    return (lib.tattn_bwd_preprocess(*pre_args, stream) or lib.tattn_bwd_dkdv(*dkdv_args, kid, stream)
+                            or lib.tattn_bwd_dq(*dq_args, qid, stream))
+
+                on = torch.cuda.current_stream(q.device)
+                _whole_wins[tune_key] = _launches_ms(one, on) <= _launches_ms(three, on)
+                if _whole_wins[tune_key]:  # as later calls run it
+                    _lib.check(one(), "tattn_bwd")
+                    return dq, dk, dv
         _lib.check(lib.tattn_bwd_dkdv(*dkdv_args, kid, stream), "tattn_bwd_dkdv")
         _lib.check(lib.tattn_bwd_dq(*dq_args, qid, stream), "tattn_bwd_dq")
     return dq, dk, dv
