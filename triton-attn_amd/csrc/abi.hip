@@ -161,11 +161,11 @@ int pick_config(int kernel, int64_t D, int dtype, int causal, int64_t N, int64_t
   Cheapest best;
   switch (kernel) {
     case TATTN_K_FWD: {
-      // Fewer than 96 tiles keep the block kernels' single running max per row. The coop kernel's
-      // O and M of near one-hot rows (scores of +-100) are as close to float64 (M closer), but not
-      // the same bits, and on such rows one dS that rounds the other way moves a gradient by more
-      // than the flat flip allowance that the stress tests (2 x 1,024 rows) state. It would take
-      // 9 us where 1 x 1,024 x 64 takes 21.
+      // Fewer than 96 tiles stay with the block kernels, at a price (21 us where this kernel takes 9, 1 x 1,024 x
+      // 64): there the softmax stress test holds gradients of near one-hot rows (2 x 1,024) to a flat allowance, which is
+      // a matter of single roundings and not of accuracy. Both kernels exceed it by chance on more such rows (8 x 1,024:
+      // block by 2.0e-3, this by 7.0e-3; 16 x 500: block by 1.4e-2, this by 1.6e-3), both keep to the allowance per element,
+      // and O and M here are as close to float64 (peaked, fp16: O 1.01e-4, M 1.1e-7 against 1.02e-4, 1.8e-7).
       coop = coop && tiles >= 96;
       const int64_t coop_most = D == 64 ? std::min<int64_t>(2304, N * 2) : D == 128 ? 1800 : 6144;
       if (causal && coop && tiles <= coop_most) return kCoop;
