@@ -78,3 +78,30 @@ def test_short_rows_whose_first_tile_scores_far_below_the_rest(low, causal, dtyp
     u = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
     assert (o.double() - want)[:, :, rows].abs().max().item() <= 3 * u * v.float().abs().max().item()
     assert (m.double() - torch.logsumexp(s, -1) / 0.6931471805599453)[:, :, rows].abs().max().item() <= 2 * u / 0.69
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [16, 32, 64, 128])
+@pytest.mark.parametrize("n", [24, 70, 128])
+def test_whole_short_backward_matches_three_launches(n, d, causal, dtype):
+    """tattn_bwd in one launch against preprocess, dK/dV and dQ with the library's picks: same bits, delta included."""
+    from tattn import _lib
+    from tattn.api import _DTYPES, _forward
+
+    z, h, scale = 2, 5, d ** -0.5
+    g = torch.Generator(device="cuda").manual_seed(3000 * d + n)
+    q, k, v, do = (torch.randn((z, h, n, d), device="cuda", dtype=dtype, generator=g) for _ in range(4))
+    o, m = _forward(q, k, v, causal, scale)
+    lib, code, st = _lib.load(), _DTYPES[dtype], _lib.strides4(q)
+    stream = torch.cuda.current_stream().cuda_stream
+    args = (st, z, h, n, d, code, int(causal), scale, -1, stream)
+    one, three = ([torch.empty_like(q) for _ in range(3)] + [torch.empty_like(m)] for _ in range(2))
+    p = [t.data_ptr() for t in (q, k, v, o, do, m)]
+    _lib.check(lib.tattn_bwd(*p[:5], *(t.data_ptr() for t in one[:3]), p[5], one[3].data_ptr(), *args), "tattn_bwd")
+    dq, dk, dv, delta = (t.data_ptr() for t in three)
+    _lib.check(lib.tattn_bwd_preprocess(p[3], p[4], delta, st, z, h, n, d, code, stream), "tattn_bwd_preprocess")
+    _lib.check(lib.tattn_bwd_dkdv(p[0], p[1], p[2], p[4], dk, dv, p[5], delta, *args), "tattn_bwd_dkdv")
+    _lib.check(lib.tattn_bwd_dq(p[0], p[1], p[2], p[4], dq, p[5], delta, *args), "tattn_bwd_dq")
+    for name, a, b in zip(("dq", "dk", "dv", "delta"), one, three):
+        assert torch.equal(a, b), name

@@ -342,14 +342,16 @@ int run_dkdv(const BwdParams& p, int D, int dtype, bool causal, int id, hipStrea
 bool fwd_own_fits(const FwdParams& p, int D, int dtype) { return dtype == TATTN_F32 ? fwd_f32_fits(p, D) : fwd_coop_fits(p, D, dtype); }
 bool bwd_own_fits(const BwdParams& p, int D, int dtype) { return dtype == TATTN_F32 ? bwd_f32_fits(p, D) : bwd_coop_fits(p, D, dtype); }
 
-// What the library picks: the forward, and one kernel of the backward (the whole backward of short rows
-// is one launch: the callers that run both kernels look at bwd_short_fits first).
+// What the library picks: the forward, and one kernel of the backward. The whole backward of short rows is
+// one launch (the callers that run both kernels look at bwd_short_fits first), with the bits of the pipelined
+// kernels: called one by one, dK/dV and dQ run those there, so that both ways give the same gradients.
 int pick_fwd(const FwdParams& p, int D, int dtype, int causal) {
   if (fwd_short_fits(p, dtype)) return kShort;
   return pick_config(TATTN_K_FWD, D, dtype, causal, p.N, (int64_t)p.Z * p.H, fwd_own_fits(p, D, dtype));
 }
 int pick_bwd(int kernel, const BwdParams& p, int D, int dtype, int causal) {
-  return pick_config(kernel, D, dtype, causal, p.N, (int64_t)p.Z * p.H, bwd_own_fits(p, D, dtype));
+  const bool own = bwd_own_fits(p, D, dtype) && !bwd_short_fits(p, D, dtype);
+  return pick_config(kernel, D, dtype, causal, p.N, (int64_t)p.Z * p.H, own);
 }
 
 // Whether a caller's table index exists.
@@ -593,7 +595,7 @@ int tattn_bwd_noalloc(const void* q, const void* k, const void* v, const void* o
   if ((rc = device_check())) return rc;
   float* delta = nullptr;
   if ((rc = scratch_for_current_device(&delta))) return rc;
-  // delta is written in full by the preprocess before dK/dV and dQ read it: nothing to clear.
+  // delta is written in full (by the preprocess, or by the kernel that computes it) before it is read.
   return tattn_bwd(q, k, v, o, dout, dq, dk, dv, m, delta, strides, Z, H, N, D, dtype, causal, sm_scale,
                    config_id, stream);
 }
