@@ -163,10 +163,6 @@ __global__ __launch_bounds__(RW * CS * 64, OCC) void fwd_coop_kernel(const FwdPa
 #pragma unroll
   for (int u = 0; u < DT; ++u) acc[u] = f32x16{};
 
-  // Tile t of the wave's row tile, staged in `st`. Probabilities against the running max as it
-  // stands (seeded for all waves by tile 0's row max); a lane whose 16 probabilities sum above 2^12 sends
-  // the wave through the row max and a rescale, as in fwd_pipe_kernel. Branches are one-sided
-  // (state updated first, undone inside): two-sided ones make the allocator hold two copies of it.
   // Raw scores of tile t (staged at `st`, lane addresses `off` bytes away), hidden keys at -inf scaled.
   auto scores = [&](const char* st, int off, int t) __attribute__((always_inline)) {
     f32x16 s = f32x16{};
@@ -185,6 +181,10 @@ __global__ __launch_bounds__(RW * CS * 64, OCC) void fwd_coop_kernel(const FwdPa
     for (int r = 0; r < 16; ++r) mx = __builtin_fmaxf(mx, s[r] * c);
     return max_halves(mx);
   };
+  // Tile t of the wave's row tile, staged in `st`. Probabilities against the running max as it
+  // stands (seeded for all waves by tile 0's row max); a lane whose 16 probabilities sum above 2^12 sends
+  // the wave through the row max and a rescale, as in fwd_pipe_kernel. Branches are one-sided
+  // (state updated first, undone inside): two-sided ones make the allocator hold two copies of it.
   auto tile = [&](const char* st, int t) __attribute__((always_inline)) {
     const f32x16 s = scores(st, 0, t);
     V8 x[2];
@@ -623,9 +623,6 @@ int dq_d(BwdParams p, bool causal, hipStream_t st) {
 
 template <typename T, int D>
 int dkdv_d(BwdParams p, bool causal, hipStream_t st) {
-  if constexpr (D == 128) {  // dK, dV, K and V of a tile do not fit a wave's 256 registers: never picked
-    return set_error(TATTN_E_CONFIG, "no dK/dV kernel with split queries at head dim 128");
-  } else {
   using S = Shape<D>;
   p.n_blocks = (p.N + 32 * S::RW - 1) / (32 * S::RW);
   const dim3 grid((unsigned)((int64_t)p.n_blocks * p.Z * p.H)), block(S::NW * 64);
@@ -633,22 +630,25 @@ int dkdv_d(BwdParams p, bool causal, hipStream_t st) {
   if (causal) dkdv_coop_kernel<T, D, S::RW, S::CS, OCC, true><<<grid, block, 0, st>>>(p);
   else dkdv_coop_kernel<T, D, S::RW, S::CS, OCC, false><<<grid, block, 0, st>>>(p);
   return check_launch("tattn_bwd_dkdv");
-  }
 }
 
-#define TATTN_COOP_SWITCH(FN)                                                               \
-  switch (D) {                                                                              \
-    case 16: return dtype == 0 ? FN<f16, 16>(p, causal, st) : FN<bf16, 16>(p, causal, st);   \
-    case 32: return dtype == 0 ? FN<f16, 32>(p, causal, st) : FN<bf16, 32>(p, causal, st);   \
-    case 64: return dtype == 0 ? FN<f16, 64>(p, causal, st) : FN<bf16, 64>(p, causal, st);   \
-    case 128: return dtype == 0 ? FN<f16, 128>(p, causal, st) : FN<bf16, 128>(p, causal, st); \
-  }                                                                                         \
-  return set_error(TATTN_E_ARG, "head dim must be 16, 32, 64 or 128, got %d", D);
+#define TATTN_COOP_CASE(FN, D_) \
+  case D_: return dtype == 0 ? FN<f16, D_>(p, causal, st) : FN<bf16, D_>(p, causal, st);
+#define TATTN_COOP_SWITCH(FN, CASE_128)                                                   \
+  switch (D) {                                                                          \
+    TATTN_COOP_CASE(FN, 16) TATTN_COOP_CASE(FN, 32) TATTN_COOP_CASE(FN, 64) CASE_128      \
+  }                                                                                     \
+  return set_error(TATTN_E_ARG, "%s: no kernel with split sums at head dim %d", #FN, D);
 
 }  // namespace
 
-int launch_fwd_coop(const FwdParams& p, int D, int dtype, bool causal, hipStream_t st) { TATTN_COOP_SWITCH(fwd_d) }
-int launch_dq_coop(const BwdParams& p, int D, int dtype, bool causal, hipStream_t st) { TATTN_COOP_SWITCH(dq_d) }
-int launch_dkdv_coop(const BwdParams& p, int D, int dtype, bool causal, hipStream_t st) { TATTN_COOP_SWITCH(dkdv_d) }
+int launch_fwd_coop(const FwdParams& p, int D, int dtype, bool causal, hipStream_t st) {
+  TATTN_COOP_SWITCH(fwd_d, TATTN_COOP_CASE(fwd_d, 128))
+}
+int launch_dq_coop(const BwdParams& p, int D, int dtype, bool causal, hipStream_t st) {
+  TATTN_COOP_SWITCH(dq_d, TATTN_COOP_CASE(dq_d, 128))
+}
+// Head dim 128: dK, dV, K and V of a tile do not fit a wave's 256 registers (never picked).
+int launch_dkdv_coop(const BwdParams& p, int D, int dtype, bool causal, hipStream_t st) { TATTN_COOP_SWITCH(dkdv_d, ) }
 
 }  // namespace tattn
