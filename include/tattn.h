@@ -68,8 +68,8 @@ int tattn_device_supported(void);
  * (src/tattn/api.py:78-99, src/tattn/kernels.py:57-148). Arbitrary z/h/n strides per tensor
  * (api.py:95-96); m is [Z,H,N] float32 contiguous (api.py:88), or NULL when no backward will
  * follow: the log-sum-exp is then not stored (the reference always stores it, api.py:88, 161).
- * config_id = -1 picks from the table by (D, dtype, causal, N); otherwise an index into
- * the TATTN_K_FWD table (the reference's `config=` override, api.py:69-75).
+ * config_id = -1 picks the kernel for the problem, from the table or outside it (tattn_picked);
+ * otherwise an index into the TATTN_K_FWD table (the reference's `config=` override, api.py:69-75).
  */
 int tattn_fwd(const void* q, const void* k, const void* v, void* o, float* m,
               const int64_t q_strides[4], const int64_t k_strides[4],
@@ -105,7 +105,8 @@ int tattn_bwd_dq(const void* q, const void* k, const void* v, const void* dout, 
                  int config_id, void* stream);
 
 /*
- * The whole backward in stream order: preprocess, dK/dV, dQ (src/tattn/api.py:102-146).
+ * The whole backward in stream order (preprocess, dK/dV, dQ: src/tattn/api.py:102-146), in one to
+ * three launches; the same bits as the three entry points above with the same picks.
  * delta is caller-owned float32 [Z,H,N] scratch. config_id applies to both dK/dV and dQ
  * (as the reference's `config=` does, api.py:124-145); -1 picks per kernel.
  */
@@ -118,7 +119,8 @@ int tattn_bwd(const void* q, const void* k, const void* v, const void* o, const 
  * tattn_bwd with the gradients in a layout of their own: q, k, v, o and do share `strides`, dq, dk
  * and dv share `grad_strides`. The backward then reads activations where they lie (a token-major
  * view, say) and writes contiguous gradients, where the reference first copies its inputs
- * contiguous (api.py:111). Same results bit for bit as tattn_bwd on contiguous copies.
+ * contiguous (api.py:111). Same results bit for bit as tattn_bwd on contiguous copies, unless rows
+ * overlap or lie so far apart that the launch goes to kernels that contiguous copies do not need.
  */
 int tattn_bwd_layouts(const void* q, const void* k, const void* v, const void* o, const void* dout,
                       void* dq, void* dk, void* dv, const float* m, float* delta,

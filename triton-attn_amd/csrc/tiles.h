@@ -40,7 +40,7 @@ template <typename T, int D> struct FwdTable;
   TATTN_TABLE(NAME, _Float16, D, __VA_ARGS__) \
   TATTN_TABLE(NAME, __bf16, D, __VA_ARGS__)
 
-// The picks per sequence length are measured and live in pick_config (abi.hip); entry 0 is the
+// The picks are measured and live in pick_config (abi.hip); entry 0 is the
 // pick wherever no rule names another. Kinds (`pipe`): 1 software-pipelined (32 rows per step),
 // 2 persistent (16-bit; where a problem does not meet its preconditions the pipelined kernel of
 // the same tiles runs it), 3 paired-wave backward, 0 generic. The 16-bit entries fit their
